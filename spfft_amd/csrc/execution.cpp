@@ -14,6 +14,7 @@
 #include <utility>
 #include <vector>
 
+#include "dft_kernels.hpp"
 #include "hip_check.hpp"
 #include "profiling.hpp"
 #include "spfft/exceptions.hpp"
@@ -76,15 +77,45 @@ bool disable_fast_path() {
 
 // Choice of plane kernels: SPFFT_AMD_PLANE=0 keeps the class-split kernels,
 // =1 forces the whole-plane kernels where they apply (batches), =2 the split
-// plane stage; unset, the autotuner decides. Returns -1 (tune), 0, 1 or 2. A
-// forced family skips the tuner (defaults for the other choices, nothing
-// recorded).
+// plane stage, =3 the matrix kernels; unset, the autotuner decides. Returns -1
+// (tune) or 0 to 3. A forced family skips the tuner (defaults for the other
+// choices, nothing recorded) and gives way to one that serves the shape.
 int plane_kernels_forced() {
   const char* v = std::getenv("SPFFT_AMD_PLANE");
   if (v && v[0] == '0') return 0;
   if (v && v[0] == '1') return 1;
   if (v && v[0] == '2') return 2;
+  if (v && v[0] == '3') return 3;
   return -1;
+}
+
+// Sticks per workgroup of the z kernels of length nz.
+template <typename T>
+int sticks_per_block(int nz) {
+  if (!fixed_length(nz)) return kDftSticks;
+  int S = 0, LZ = 0, shift = 0;
+  fast_z_geometry<T>(nz, &S, &LZ, &shift);
+  return S;
+}
+
+// The z stage of one transform.
+template <typename T>
+void launch_z(bool forward, int nx, int ny, int nz, const FastArgs<T>& a, hipStream_t stream) {
+  if (!fixed_length(nz)) {
+    launch_dft_z<T>(forward, nx, ny, a, stream);
+  } else if (forward) {
+    launch_fast_z_forward<T>(nz, a, stream);
+  } else {
+    launch_fast_z_backward<T>(nz, a, stream);
+  }
+}
+
+// The plane family to run for `want` among those that serve the shape: the
+// class-split kernels, else the split stage, else the matrix kernels.
+int served_plane(int want, bool classSplit, bool split, bool matrix) {
+  if (want == 3 && matrix) return 3;
+  if (want == 2 && split) return 2;
+  return classSplit ? 0 : (split ? 2 : 3);
 }
 
 // Mean time of `reps` launches after one warm-up launch, in milliseconds.
@@ -173,11 +204,22 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
   tb.allowFast = fast;
   const StickTables t = build_stick_tables(*map);
   tb.numCols = static_cast<int>(t.colX.size());
-  // fixed-length kernels when the lengths have compile-time schedules
-  tb.fast = fast && fast_path_supported<T>(map->dimX, map->dimY, map->dimZ, tb.numCols,
-                                           map->type == SPFFT_TRANS_R2C);
-  tb.classSplit = tb.fast && class_split_supported<T>(map->dimX, map->dimY, tb.numCols,
-                                                      map->type == SPFFT_TRANS_R2C);
+  const bool r2c = map->type == SPFFT_TRANS_R2C;
+  auto centred = [](int i, int n) { return std::min(i, n - i); };
+  for (int x : t.colX) tb.kx = std::max(tb.kx, centred(x, map->dimX));
+  for (int y : t.stickY) tb.ky = std::max(tb.ky, centred(y, map->dimY));
+  for (int slot : t.entrySlot) {
+    tb.kz = std::max(tb.kz, centred(slot % map->dimZ, map->dimZ));
+  }
+  // The plane stage of a set: fixed-length kernels when both lengths have
+  // compile-time schedules, matrix kernels when the plane fits them.
+  tb.split = fast && tb.numCols >= 1 && fixed_length(map->dimX) && fixed_length(map->dimY);
+  tb.matrix = fast && tb.numCols >= 1 &&
+              dft_plane_supported<T>(r2c, map->dimX, map->dimY, tb.kx, tb.ky);
+  tb.fast = z_supported(map->dimZ) && (tb.split || tb.matrix);
+  tb.fixedLengths = tb.split && fixed_length(map->dimZ);
+  tb.classSplit = tb.fast && tb.split &&
+                  class_split_supported<T>(map->dimX, map->dimY, tb.numCols, r2c);
   const bool useFast = tb.fast;
   tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
   tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
@@ -203,16 +245,38 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
       at[(static_cast<size_t>(t.stickCol[s]) * M + y % M) * R + y / M] = s;
     }
     tb.stickAt = DeviceBuffer<int>::from_host(at);
+    // tables of the matrix kernels
+    if (tb.matrix) {
+      const int nx = map->dimX;
+      std::vector<int> cell(map->num_sticks());
+      std::vector<int> columns(
+          static_cast<size_t>(dft::tile_columns(nx, tb.kx, r2c)) * ny, map->num_sticks());
+      for (int s = 0; s < map->num_sticks(); ++s) {
+        const int x = t.colX[t.stickCol[s]], y = t.stickY[s];
+        const int i = r2c ? x : dft::fold_at(nx, tb.kx, x);
+        cell[s] = i << 16 | dft::fold_at(ny, tb.ky, y);
+        columns[static_cast<size_t>(i) * ny + y] = s;
+      }
+      tb.stickCell = DeviceBuffer<int>::from_host(cell);
+      tb.columnSticks = DeviceBuffer<int>::from_host(columns);
+    }
+    if (tb.matrix || !fixed_length(map->dimZ)) {
+      const DftTables at(map->dimX, ny, map->dimZ);
+      tb.trig = DeviceBuffer<double>(2 * static_cast<size_t>(at.total));
+      build_dft_tables(tb.trig.data(), map->dimX, ny, map->dimZ, stream);
+    }
     // Entry list for the z kernels: value index and position in the LDS tile
     // of the workgroup that owns the stick; earlier copies of a repeated
     // triplet are flagged so that the last one wins on scatter.
-    int S = 0, LZ = 0, shift = 0;
-    fast_z_geometry<T>(map->dimZ, &S, &LZ, &shift);
+    int S = kDftSticks, LZ = dft::z_pitch(map->dimZ, tb.kz), shift = 0;
+    const bool fixedZ = fixed_length(map->dimZ);
+    if (fixedZ) fast_z_geometry<T>(map->dimZ, &S, &LZ, &shift);
     std::vector<int2> ent(map->num_values());
     for (int e = 0; e < map->num_values(); ++e) {
       const int slot = t.entrySlot[e];
       const int st = slot / map->dimZ, z = slot % map->dimZ;
-      int pos = (st % S) * LZ + z + (z >> shift);
+      int pos = (st % S) * LZ +
+                (fixedZ ? z + (z >> shift) : dft::fold_at(map->dimZ, tb.kz, z));
       if (e + 1 < map->num_values() && t.entrySlot[e + 1] == slot) pos |= int(0x80000000u);
       ent[e] = make_int2(t.entryValue[e], pos);
     }
@@ -354,6 +418,8 @@ ExecutionGPU<T>::ExecutionGPU(const std::shared_ptr<IndexMap>& map,
   numCols_ = tab_->numCols;
   fast_ = tab_->fast;
   classSplit_ = tab_->classSplit;
+  split_ = tab_->split;
+  matrix_ = tab_->matrix;
   pitchT_ = tab_->pitchT;
 
   fftX_ = make_fft_desc(map_->dimX);
@@ -425,13 +491,14 @@ FastArgs<T> ExecutionGPU<T>::fast_args() const {
   a.nst = map_->num_sticks();
   a.ncol = numCols_;
   a.zbuf = reinterpret_cast<Cx<T>*>(grid_->sticks_gpu());
-  a.entryValue = tab_->entryValue.data();
-  a.entrySlot = tab_->entrySlot.data();
+  a.kx = tab_->kx;
+  a.ky = tab_->ky;
+  a.kz = tab_->kz;
+  a.stickCell = tab_->stickCell.data();
+  a.columnSticks = tab_->columnSticks.data();
+  a.trig = tab_->trig.data();
   a.stickBegin = tab_->stickBegin.data();
-  a.stickY = tab_->stickY.data();
-  a.stickCol = tab_->stickCol.data();
   a.colX = tab_->colX.data();
-  a.colBegin = tab_->colBegin.data();
   a.stickAt = tab_->stickAt.data();
   a.zEntries = tab_->zEntries.data();
   a.pitch = fast_pitch<T>(map_->num_sticks());
@@ -463,33 +530,29 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
                                           bool staged) {
   TuneChoice c;
   c.zRuns = f.hasRuns;
-  const bool classSplit = classSplit_;
   const int forced = plane_kernels_forced();
-  if (forced >= 0 || !classSplit) {
-    // single transforms have no whole-plane kernels; x != y planes and
-    // lengths without class-split kernels only the split stage
-    c.plane = forced == 2 || !classSplit ? 2 : 0;
-    if (forced >= 0) return c;
-  }
+  // single transforms have no whole-plane kernels; x != y planes and lengths
+  // without class-split kernels only the split stage and the matrix kernels,
+  // lengths that are not fixed only the latter
+  c.plane = served_plane(forced, classSplit_, split_, matrix_);
+  if (forced >= 0) return c;
   // batched fallbacks on the transform's own stream keep the defaults
   if (stream != nullptr) return c;
+  const bool fixedZ = fixed_length(map_->dimZ);
+  // nothing to choose
+  if (!split_ && !(fixedZ && f.hasRuns)) return c;
   const TuneKey key = make_tune_key(grid_->device_id(), static_cast<int>(sizeof(T)), map_->dimX,
                                     map_->dimY, map_->dimZ, map_->type == SPFFT_TRANS_R2C,
-                                    forward, numCols_, 1);
-  if (tune_lookup(key, &c)) {
-    c.zRuns = c.zRuns && f.hasRuns;
-    if (c.plane == 1) c.plane = 0;
-    if (!classSplit) c.plane = 2;
+                                    forward, numCols_, map_->num_sticks(), 1);
+  TuneChoice known;
+  if (tune_lookup(key, &known)) {
+    c.zRuns = known.zRuns && f.hasRuns;
+    c.plane = served_plane(known.plane, classSplit_, split_, matrix_);
     return c;
   }
   // Host data staged in the work buffer, which the split stage's candidate
   // launches would overwrite: no timing on this call (defaults).
-  if (staged) {
-    c = TuneChoice();
-    c.zRuns = f.hasRuns;
-    c.plane = classSplit ? 0 : 2;
-    return c;
-  }
+  if (staged) return c;
   // Every launch below is idempotent: backward z reads the values and writes
   // the [z][stick] buffer, the plane stage reads that buffer and writes the
   // output; forward the plane stage reads the input and writes the buffer,
@@ -500,11 +563,7 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   a.nz = map_->dimZ;
   auto z = [&](int runs) {
     a.hasRuns = runs;
-    if (forward) {
-      launch_fast_z_forward<T>(map_->dimZ, a, nullptr);
-    } else {
-      launch_fast_z_backward<T>(map_->dimZ, a, nullptr);
-    }
+    launch_z<T>(forward, map_->dimX, map_->dimY, map_->dimZ, a, nullptr);
   };
   auto xy_fused = [&] {
     if (forward) {
@@ -514,24 +573,30 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     }
   };
   auto xy_two = [&] { launch_split_xy<T>(forward, map_->dimX, map_->dimY, a, nullptr); };
-  float zr = 0.f, ze = 0.f, fused = 0.f, two = 0.f;
+  auto xy_matrix = [&] { launch_dft_xy<T>(forward, map_->dimX, map_->dimY, a, nullptr); };
+  float zr = 0.f, ze = 0.f, fused = 0.f, two = 0.f, matrix = 0.f;
   auto time_z = [&] {
-    if (f.hasRuns) {
+    if (f.hasRuns && fixedZ) {
       zr = time_launches([&] { z(1); }, ev.e0, ev.e1);
       ze = time_launches([&] { z(0); }, ev.e0, ev.e1);
       c.zRuns = zr <= ze ? 1 : 0;
     } else {
-      z(0);
+      z(f.hasRuns);
     }
   };
   auto time_xy = [&] {
-    two = time_launches(xy_two, ev.e0, ev.e1);
-    if (classSplit) {
-      fused = time_launches(xy_fused, ev.e0, ev.e1);
-      c.plane = two < fused ? 2 : 0;
-    } else {
-      c.plane = 2;
-    }
+    float best = 0.f;
+    auto candidate = [&](bool serves, int plane, float* ms, auto&& run) {
+      if (!serves) return;
+      *ms = time_launches(run, ev.e0, ev.e1);
+      if (best == 0.f || *ms < best) {
+        best = *ms;
+        c.plane = plane;
+      }
+    };
+    candidate(classSplit_, 0, &fused, xy_fused);
+    candidate(split_, 2, &two, xy_two);
+    candidate(matrix_, 3, &matrix, xy_matrix);
   };
   if (forward) {
     time_xy();
@@ -543,10 +608,11 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   tune_record(key, c);
   if (tune_log_enabled()) {
     std::fprintf(stderr, "spfft_amd tune: %s N=%d Nz=%d %s %s, single transform, %d columns: z "
-                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f ms -> plane=%d "
-                 "zruns=%d\n", sizeof(T) == 8 ? "double" : "float", map_->dimX, map_->dimZ,
-                 map_->type == SPFFT_TRANS_R2C ? "R2C" : "C2C", forward ? "forward" : "backward",
-                 numCols_, zr, ze, fused, two, c.plane, c.zRuns);
+                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f, matrix %.4f ms -> "
+                 "plane=%d zruns=%d\n", sizeof(T) == 8 ? "double" : "float", map_->dimX,
+                 map_->dimZ, map_->type == SPFFT_TRANS_R2C ? "R2C" : "C2C",
+                 forward ? "forward" : "backward", numCols_, zr, ze, fused, two, matrix, c.plane,
+                 c.zRuns);
   }
   return c;
 }
@@ -687,13 +753,15 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent) {
     const TuneChoice choice =
         single_choice(false, f, stream, inKind != MemKind::Device || hostOut);
     f.hasRuns = choice.zRuns;
-    launch_fast_z_backward<T>(map_->dimZ, f, stream);
+    launch_z<T>(false, map_->dimX, map_->dimY, map_->dimZ, f, stream);
     // host output: the plane stage runs in chunks of planes, each copied out
     // while the next is computed
     for (int c = 0; c < chunks; ++c) {
       f.zBegin = c * ppc;
       f.nz = std::min(map_->dimZ, (c + 1) * ppc);
-      if (choice.plane == 2) {
+      if (choice.plane == 3) {
+        launch_dft_xy<T>(false, map_->dimX, map_->dimY, f, stream);
+      } else if (choice.plane == 2) {
         launch_split_xy<T>(false, map_->dimX, map_->dimY, f, stream);
       } else {
         launch_fast_xy_backward<T>(map_->dimX, map_->dimY, f, stream);
@@ -778,7 +846,9 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
       if (hostIn) upload_chunk(c);
       f.zBegin = c * ppc;
       f.nz = std::min(map_->dimZ, (c + 1) * ppc);
-      if (choice.plane == 2) {
+      if (choice.plane == 3) {
+        launch_dft_xy<T>(true, map_->dimX, map_->dimY, f, stream);
+      } else if (choice.plane == 2) {
         launch_split_xy<T>(true, map_->dimX, map_->dimY, f, stream);
       } else {
         launch_fast_xy_forward<T>(map_->dimX, map_->dimY, f, stream);
@@ -787,7 +857,7 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
     f.zBegin = 0;
     f.nz = map_->dimZ;
     f.hasRuns = choice.zRuns;
-    launch_fast_z_forward<T>(map_->dimZ, f, stream);
+    launch_z<T>(true, map_->dimX, map_->dimY, map_->dimZ, f, stream);
   } else {
     if (hostIn) {
       for (int c = 0; c < chunks; ++c) upload_chunk(c);
@@ -858,14 +928,22 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
     din[t] = i.second;
     dout[t] = o.second;
   }
-  int S = 0, LZ = 0, shift = 0;
-  fast_z_geometry<T>(m0.dimZ, &S, &LZ, &shift);
+  const int S = sticks_per_block<T>(m0.dimZ);
   shape->blocks = 0;
   shape->maxNcol = 0;
   shape->runs = true;
-  shape->classSplit = true;
+  shape->classSplit = shape->split = shape->matrix = shape->fixedLengths = true;
+  shape->maxNst = shape->kx = shape->ky = shape->kz = 0;
   for (size_t t = 0; t < n; ++t) {
+    const TransformTables<T>& tab = *ex[t]->tab_;
     shape->classSplit = shape->classSplit && ex[t]->classSplit_;
+    shape->split = shape->split && ex[t]->split_;
+    shape->matrix = shape->matrix && ex[t]->matrix_;
+    shape->fixedLengths = shape->fixedLengths && tab.fixedLengths;
+    shape->maxNst = std::max(shape->maxNst, ex[t]->map_->num_sticks());
+    shape->kx = std::max(shape->kx, tab.kx);
+    shape->ky = std::max(shape->ky, tab.ky);
+    shape->kz = std::max(shape->kz, tab.kz);
     shape->blocks += (ex[t]->map_->num_sticks() + S - 1) / S;
     shape->maxNcol = std::max(shape->maxNcol, ex[t]->numCols_);
     shape->runs = shape->runs && ex[t]->tab_->zInfo.data() != nullptr;
@@ -875,7 +953,10 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
   shape->dimY = m0.dimY;
   shape->dimZ = m0.dimZ;
   shape->device = ex[0]->grid_->device_id();
-  return true;
+  // the widest columns of different transforms together must fit as well
+  shape->matrix = shape->matrix &&
+                  dft_plane_supported<T>(shape->r2c, m0.dimX, m0.dimY, shape->kx, shape->ky);
+  return shape->split || shape->matrix;
 }
 
 template <typename T>
@@ -883,7 +964,7 @@ bool ExecutionGPU<T>::plane_candidate(ExecutionGPU<T>* const* ex, size_t n, cons
                                       T* const* dout, bool forward, const BatchShape& shape) {
   // whole-plane kernels are a candidate when every transform has its tile
   // positions and the widest tile fits
-  bool ok = plane_kernels_forced() != 0 && shape.dimX == shape.dimY &&
+  bool ok = plane_kernels_forced() != 0 && shape.split && shape.dimX == shape.dimY &&
             plane_path_supported<T>(shape.dimX, shape.maxNcol, shape.r2c);
   for (size_t t = 0; t < n && ok; ++t) ok = ex[t]->pitchT_ > 0;
   // The FP32 whole-plane kernels move two elements per 16-byte access, so
@@ -901,8 +982,7 @@ void ExecutionGPU<T>::fill_batch_tables(ExecutionGPU<T>* const* ex, size_t n, co
                                         T* const* dout, bool forward,
                                         const SpfftScalingType* scaling, FastArgs<T>* args,
                                         int2* zmap) {
-  int S = 0, LZ = 0, shift = 0;
-  fast_z_geometry<T>(ex[0]->map_->dimZ, &S, &LZ, &shift);
+  const int S = sticks_per_block<T>(ex[0]->map_->dimZ);
   size_t k = 0;
   for (size_t t = 0; t < n; ++t) {
     FastArgs<T> f = ex[t]->fast_args();
@@ -917,11 +997,27 @@ void ExecutionGPU<T>::fill_batch_tables(ExecutionGPU<T>* const* ex, size_t n, co
 }
 
 template <typename T>
+void ExecutionGPU<T>::launch_batch_z(bool forward, const BatchShape& shape, bool runs,
+                                     const FastArgs<T>* dArgs, const int2* dMap,
+                                     hipStream_t stream) {
+  if (fixed_length(shape.dimZ)) {
+    launch_fast_z_batch<T>(forward, shape.r2c, shape.dimZ, dArgs, dMap, shape.blocks, runs,
+                           stream);
+  } else {
+    launch_dft_z_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, shape.dimZ, shape.kz, dArgs,
+                          dMap, shape.blocks, runs, stream);
+  }
+}
+
+template <typename T>
 void ExecutionGPU<T>::launch_batch(bool forward, const BatchShape& shape, int n,
                                    const TuneChoice& choice, const FastArgs<T>* dArgs,
                                    const int2* dMap, hipStream_t stream) {
   auto launch_xy = [&] {
-    if (choice.plane == 2) {
+    if (choice.plane == 3) {
+      launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, shape.kx, shape.ky,
+                             dArgs, n, shape.dimZ, stream);
+    } else if (choice.plane == 2) {
       launch_split_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, dArgs, n, shape.dimZ,
                                shape.maxNcol, stream);
     } else if (choice.plane == 1) {
@@ -932,14 +1028,9 @@ void ExecutionGPU<T>::launch_batch(bool forward, const BatchShape& shape, int n,
                               shape.maxNcol, stream);
     }
   };
-  const bool runs = choice.zRuns != 0;
-  if (forward) {
-    launch_xy();
-    launch_fast_z_batch<T>(true, shape.r2c, shape.dimZ, dArgs, dMap, shape.blocks, runs, stream);
-  } else {
-    launch_fast_z_batch<T>(false, shape.r2c, shape.dimZ, dArgs, dMap, shape.blocks, runs, stream);
-    launch_xy();
-  }
+  if (forward) launch_xy();
+  launch_batch_z(forward, shape, choice.zRuns != 0, dArgs, dMap, stream);
+  if (!forward) launch_xy();
 }
 
 template <typename T>
@@ -948,8 +1039,7 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
   TuneChoice c;
   TuneEvents ev;
   auto z = [&](bool runs) {
-    launch_fast_z_batch<T>(forward, shape.r2c, shape.dimZ, dArgs, dMap, shape.blocks, runs,
-                           nullptr);
+    launch_batch_z(forward, shape, runs, dArgs, dMap, nullptr);
   };
   auto xy_split = [&] {
     launch_fast_xy_batch<T>(forward, shape.r2c, shape.dimX, dArgs, n, shape.dimZ, shape.maxNcol,
@@ -963,13 +1053,19 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
     launch_split_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, dArgs, n, shape.dimZ,
                              shape.maxNcol, nullptr);
   };
+  auto xy_matrix = [&] {
+    launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, shape.kx, shape.ky, dArgs,
+                           n, shape.dimZ, nullptr);
+  };
   // The forward z kernel reads the [z][stick] buffer that the xy kernel
   // writes, the backward xy kernel the one that the z kernel writes.
   if (forward) {
     if (shape.classSplit) {
       xy_split();
-    } else {
+    } else if (shape.split) {
       xy_two();
+    } else {
+      xy_matrix();
     }
   }
   float zr = 0.f, ze = 0.f;
@@ -980,10 +1076,19 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
   } else if (!forward) {
     z(false);
   }
-  float split = 0.f, plane0 = 0.f, plane1 = 0.f, two = 0.f;
-  two = time_launches(xy_two, ev.e0, ev.e1);
-  float best = two;
-  c.plane = 2;
+  float split = 0.f, plane0 = 0.f, plane1 = 0.f, two = 0.f, matrix = 0.f;
+  float best = 1e30f;
+  if (shape.matrix) {
+    best = matrix = time_launches(xy_matrix, ev.e0, ev.e1);
+    c.plane = 3;
+  }
+  if (shape.split) {
+    two = time_launches(xy_two, ev.e0, ev.e1);
+    if (two <= best) {
+      best = two;
+      c.plane = 2;
+    }
+  }
   if (shape.classSplit) {
     // x != y planes and lengths without class-split kernels have the split
     // stage only
@@ -1013,10 +1118,10 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
     std::fprintf(stderr,
                  "spfft_amd tune: %s N=%d Nz=%d %s %s, %d transforms, %d columns: z runs %.3f / "
                  "entries %.3f ms; class-split %.3f, split stage %.3f, whole-plane %.3f, one per "
-                 "CU %.3f ms -> plane=%d slots=%d zruns=%d\n",
+                 "CU %.3f, matrix %.3f ms -> plane=%d slots=%d zruns=%d\n",
                  sizeof(T) == 8 ? "double" : "float", shape.dimX, shape.dimZ,
                  shape.r2c ? "R2C" : "C2C", forward ? "forward" : "backward", n, shape.maxNcol,
-                 zr, ze, split, two, plane0, plane1, c.plane, c.slots, c.zRuns);
+                 zr, ze, split, two, plane0, plane1, matrix, c.plane, c.slots, c.zRuns);
   }
   return c;
 }
@@ -1088,10 +1193,12 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   const int forced = plane_kernels_forced();
   if (forced >= 0) {
     choice.plane = forced;
+  } else if (!shape.split && !(fixed_length(shape.dimZ) && shape.runs)) {
+    choice.plane = 3;  // nothing to choose
   } else {
     const TuneKey tkey = make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
                                        shape.dimY, shape.dimZ, shape.r2c, forward,
-                                       shape.maxNcol, nt);
+                                       shape.maxNcol, shape.maxNst, nt);
     if (!tune_lookup(tkey, &choice)) {
       choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap);
       tune_record(tkey, choice);
@@ -1101,7 +1208,9 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
     choice.plane = 0;
     choice.slots = 0;
   }
-  if (choice.plane == 0 && !shape.classSplit) choice.plane = 2;
+  if (choice.plane != 1) {
+    choice.plane = served_plane(choice.plane, shape.classSplit, shape.split, shape.matrix);
+  }
   if (plan.exec && (plan.choice.plane != choice.plane || plan.choice.slots != choice.slots ||
                     plan.choice.zRuns != choice.zRuns)) {
     (void)hipGraphExecDestroy(plan.exec);
@@ -1151,7 +1260,9 @@ void ExecutionGPU<T>::run_batch_noalloc(ExecutionGPU<T>* const* ex, size_t n, co
   const T** din = reinterpret_cast<const T**>(h);
   T** dout = reinterpret_cast<T**>(h + n * sizeof(void*));
   BatchShape shape;
-  if (!batch_qualifies(ex, n, in, out, din, dout, &shape)) throw InvalidParameterError();
+  if (!batch_qualifies(ex, n, in, out, din, dout, &shape) || !shape.fixedLengths) {
+    throw InvalidParameterError();
+  }
   const size_t argBytes = (n * sizeof(FastArgs<T>) + 255) / 256 * 256;
   const size_t tableBytes = argBytes + static_cast<size_t>(shape.blocks) * sizeof(int2);
   if (tableBytes > scratchBytes || viewBytes + tableBytes > stageBytes) {
@@ -1171,14 +1282,16 @@ void ExecutionGPU<T>::run_batch_noalloc(ExecutionGPU<T>* const* ex, size_t n, co
   } else {
     (void)tune_recorded(make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
                                       shape.dimY, shape.dimZ, shape.r2c, forward, shape.maxNcol,
-                                      static_cast<int>(n)),
+                                      shape.maxNst, static_cast<int>(n)),
                         &choice);
   }
   if (choice.plane == 1 && !plane_candidate(ex, n, din, dout, forward, shape)) {
     choice.plane = 0;
     choice.slots = 0;
   }
-  if (choice.plane == 0 && !shape.classSplit) choice.plane = 2;
+  if (choice.plane != 1) {
+    choice.plane = served_plane(choice.plane, shape.classSplit, shape.split, shape.matrix);
+  }
   const auto* dArgs = static_cast<const FastArgs<T>*>(scratch);
   const auto* dMap = reinterpret_cast<const int2*>(static_cast<const char*>(scratch) + argBytes);
   launch_batch(forward, shape, static_cast<int>(n), choice, dArgs, dMap, nullptr);

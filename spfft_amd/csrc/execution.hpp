@@ -29,8 +29,12 @@ struct TransformTables {
   std::shared_ptr<const IndexMap> map;
   int device = 0;
   bool allowFast = true;  // built with the fixed-length path allowed
-  bool fast = false;      // fixed-length kernels serve this set
-  bool classSplit = false;  // and the class-split plane kernels (nx = ny, LDS fits)
+  bool fast = false;      // fixed-length or matrix kernels serve this set
+  bool split = false;     // the split plane stage does (fixed Nx and Ny)
+  bool matrix = false;    // the matrix plane kernels do
+  bool classSplit = false;    // the class-split plane kernels do (nx = ny, LDS fits)
+  bool fixedLengths = false;  // all three lengths are fixed ones
+  int kx = 0, ky = 0, kz = 0;  // largest centred index per dimension
   int numCols = 0;
   int pitchT = 0;  // whole-plane batch kernels' tile pitch (0: not applicable)
   DeviceBuffer<Tw<T>> twX, twY, twZ;
@@ -38,6 +42,8 @@ struct TransformTables {
   DeviceBuffer<int> stickAt;
   DeviceBuffer<int2> zEntries;
   DeviceBuffer<int4> zInfo;  // stick runs, when every stick is one run in user order
+  DeviceBuffer<int> stickCell, columnSticks;  // matrix plane kernels
+  DeviceBuffer<double> trig;                  // matrix kernels
   DeviceBuffer<int> resSticks, resBegin, xCol, resYM;
 };
 
@@ -63,8 +69,8 @@ public:
   void synchronize(SpfftExecType mode, bool concurrent = false);
 
   // Batched execution of several transforms of one shape on the fixed-length
-  // path: one z launch and one xy launch for the whole batch, on the default
-  // stream. The argument tables and the captured launch chain (a HIP graph)
+  // or matrix kernels: one z launch and one xy launch (two for the split stage)
+  // for the whole batch, on the default stream. The argument tables and the captured launch chain (a HIP graph)
   // are kept for the most recent batches and replayed when the same
   // transforms are called again with the same pointers. Returns false without
   // doing anything when the batch does not qualify (different shapes,
@@ -82,6 +88,10 @@ public:
     int dimX = 0, dimY = 0, dimZ = 0;
     bool runs = false;  // every transform's sticks are runs in user order
     bool classSplit = false;  // class-split plane kernels serve every transform
+    bool split = false, matrix = false;  // the split stage, the matrix kernels do
+    bool fixedLengths = false;           // all lengths are fixed ones
+    int maxNst = 0;                      // most sticks
+    int kx = 0, ky = 0, kz = 0;          // largest centred indices
     int device = 0;
   };
   // True when the n transforms can run as one fused chain; then din/dout (n
@@ -96,6 +106,9 @@ public:
   static void fill_batch_tables(ExecutionGPU* const* ex, size_t n, const T* const* din,
                                 T* const* dout, bool forward, const SpfftScalingType* scaling,
                                 FastArgs<T>* args, int2* zmap);
+  // The z launch of the fused chain (runs: sticks addressed as runs).
+  static void launch_batch_z(bool forward, const BatchShape& shape, bool runs,
+                             const FastArgs<T>* dArgs, const int2* dMap, hipStream_t stream);
   // The fused chain with the given kernel choices (choice.plane is honoured
   // only when the whole-plane kernels can serve the batch).
   static void launch_batch(bool forward, const BatchShape& shape, int n, const TuneChoice& choice,
@@ -152,8 +165,8 @@ private:
                 const hipEvent_t* ready, int readyCount, hipStream_t compute, hipStream_t copy);
   StageArgs<T> base_args() const;
   FastArgs<T> fast_args() const;
-  // Kernel choices of a single transform (plane stage: class-split or split
-  // kernels; z addressing when the sticks are runs), tuned on the first call
+  // Kernel choices of a single transform (plane stage: class-split, split or
+  // matrix kernels; z addressing when the sticks are runs), tuned on the first call
   // of the shape with device input and output, on that call's buffers
   // (staged = host data in the work buffer: recorded choices or defaults).
   TuneChoice single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream, bool staged);
@@ -168,9 +181,9 @@ private:
   int zBatch_ = 1, yBatch_ = 1, xBatch_ = 1;
   FftDesc fftX_, fftY_, fftZ_;
   std::shared_ptr<TransformTables<T>> tab_;  // shared with transforms of the same set
-  // fixed-length path (two kernels per direction)
+  // fixed-length and matrix kernels (two or three launches per direction)
   bool fast_ = false;
-  bool classSplit_ = false;  // class-split plane kernels too (else the split stage only)
+  bool classSplit_ = false, split_ = false, matrix_ = false;  // plane families that serve the set
   // whole-plane batch kernels (power-of-two lengths up to 128, C2C): tile pitch
   int pitchT_ = 0;
   // host I/O (created on the first call with a host pointer): chunk-ready

@@ -17,6 +17,7 @@
 #include <type_traits>
 #include <unordered_map>
 
+#include "device_args.hpp"
 #include "fast_kernels.hpp"
 #include "fft_common.hpp"
 #include "hip_check.hpp"
@@ -375,25 +376,6 @@ constexpr int round_up(int n, int m) { return (n + m - 1) / m * m; }
 template <typename T>
 __host__ __device__ constexpr int tw_offset(int n) {
   return round_up(n, static_cast<int>(sizeof(Tw<T>) / sizeof(Cx<T>)));
-}
-
-// Element `i` of an array smaller than 4 GiB, addressed with a 32-bit byte
-// offset (lets the compiler use a scalar base and one offset register).
-template <typename X>
-__device__ __forceinline__ X at32(const X* base, int i) {
-  const unsigned off = static_cast<unsigned>(i) * static_cast<unsigned>(sizeof(X));
-  return *reinterpret_cast<const X*>(reinterpret_cast<const char*>(base) + off);
-}
-
-// Workgroup barrier for LDS data: waits for this wave's LDS operations only.
-// __syncthreads() releases at workgroup scope for all memory, which waits for
-// every global load and store in flight (loads issued ahead of the barrier
-// would land before it). No kernel here passes data between waves through
-// global memory.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Streaming store (no cache allocation on the way to HBM): for batch outputs
@@ -1855,43 +1837,6 @@ __device__ __forceinline__ void full_rows(const FastArgs<T>& a, int z, int line,
   for (int e = 0; e < L::E; ++e) v[e] = in[q + L::P * e];
 }
 
-// Arguments read from a device table hold generic pointers, so the compiler
-// would access them with flat instructions (which share the LDS counter and
-// serialise against LDS traffic). Rebasing each pointer on a kernel argument
-// (a global pointer) keeps the address and lets the accesses be global ones.
-// A null pointer stays null (no offset is formed from it).
-template <typename P>
-__device__ __forceinline__ P* rebase(const char* anchor, P* p) {
-  if (p == nullptr) return nullptr;
-  return (P*)(anchor + (reinterpret_cast<const char*>(p) - anchor));
-}
-template <typename T>
-__device__ __forceinline__ FastArgs<T> on_global(FastArgs<T> a, const void* table) {
-  const char* g = static_cast<const char*>(table);
-  a.zbuf = rebase(g, a.zbuf);
-  a.in = rebase(g, a.in);
-  a.out = rebase(g, a.out);
-  a.entryValue = rebase(g, a.entryValue);
-  a.entrySlot = rebase(g, a.entrySlot);
-  a.stickBegin = rebase(g, a.stickBegin);
-  a.stickY = rebase(g, a.stickY);
-  a.stickCol = rebase(g, a.stickCol);
-  a.colX = rebase(g, a.colX);
-  a.colBegin = rebase(g, a.colBegin);
-  a.stickAt = rebase(g, a.stickAt);
-  a.zEntries = rebase(g, a.zEntries);
-  a.zInfo = rebase(g, a.zInfo);
-  a.xCol = rebase(g, a.xCol);
-  a.resSticks = rebase(g, a.resSticks);
-  a.resBegin = rebase(g, a.resBegin);
-  a.resYM = rebase(g, a.resYM);
-  a.ybuf = rebase(g, a.ybuf);
-  a.twX = rebase(g, a.twX);
-  a.twY = rebase(g, a.twY);
-  a.twZ = rebase(g, a.twZ);
-  return a;
-}
-
 // ---- entry points: one transform (arguments by value) or a batch of
 // transforms of one shape (argument table in device memory). A batched z
 // launch maps each workgroup to (transform, block) through `map`; a batched
@@ -2299,10 +2244,8 @@ bool fits(int ncol, bool rc) {
          XYShape<T, N>::lds_forward() <= kLdsMax;
 }
 
-// Lengths with class-split (and, for some, whole-plane) kernels, and all
-// lengths with z and split-stage kernels.
+// Lengths with class-split (and, for some, whole-plane) kernels.
 bool square_length(int n) { return n == 32 || n == 64 || n == 96 || n == 128 || n == 192; }
-bool fast_length(int n) { return square_length(n) || split_only_length(n); }
 
 #define SPFFT_SQUARE_SWITCH(N, CALL) \
   switch (N) {                       \
@@ -2418,13 +2361,6 @@ void fast_z_geometry(int nz, int* sticksPerBlock, int* lineLength, int* padShift
   *sticksPerBlock = g[0];
   *lineLength = g[1];
   *padShift = g[2];
-}
-
-template <typename T>
-bool fast_path_supported(int nx, int ny, int nz, int ncol, bool r2c) {
-  (void)r2c;
-  // the z kernels and the split plane stage serve every fast length
-  return fast_length(nx) && fast_length(ny) && fast_length(nz) && ncol >= 1;
 }
 
 template <typename T>
@@ -2794,7 +2730,6 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
   template int fast_xy_pitch_a<T>(int, int);                                             \
   template void launch_fast_xy_batch<T>(bool, bool, int, const FastArgs<T>*, int, int,   \
                                         int, hipStream_t);                               \
-  template bool fast_path_supported<T>(int, int, int, int, bool);                        \
   template bool class_split_supported<T>(int, int, int, bool);                           \
   template void launch_fast_xy_backward<T>(int, int, const FastArgs<T>&, hipStream_t);   \
   template void launch_fast_xy_forward<T>(int, int, const FastArgs<T>&, hipStream_t);
@@ -2807,6 +2742,7 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
 #define SPFFT_FAST_UNIT 0
 #endif
 #if SPFFT_FAST_UNIT == 0
+bool fixed_length(int n) { return square_length(n) || split_only_length(n); }
 SPFFT_INSTANTIATE_FAST_PLANE(double)
 #elif SPFFT_FAST_UNIT == 1
 SPFFT_DEFINE_GROUP(z_group0, ZCall, double, SPFFT_Z_CASE, SPFFT_LENGTHS_0)

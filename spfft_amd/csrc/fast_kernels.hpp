@@ -48,13 +48,15 @@ struct FastArgs {
   Cx<T>* zbuf = nullptr;
   const T* in = nullptr;
   T* out = nullptr;
-  const int* entryValue = nullptr;
-  const int* entrySlot = nullptr;
+  // matrix kernels (dft_kernels.hpp): largest centred |x|, |y|, |z| of the set;
+  // per stick tile column << 16 | folded y; stick index (or nst) at [tile
+  // column][y]; trig tables
+  int kx = 0, ky = 0, kz = 0;
+  const int* stickCell = nullptr;
+  const int* columnSticks = nullptr;
+  const void* trig = nullptr;
   const int* stickBegin = nullptr;
-  const int* stickY = nullptr;
-  const int* stickCol = nullptr;
   const int* colX = nullptr;
-  const int* colBegin = nullptr;
   const int* stickAt = nullptr;       // [ncol + 1][M][R]: stick index at (column, y = j + M l),
                                       // or nst (the zero element); row ncol is all nst
   const int2* zEntries = nullptr;     // per value (sorted by slot): {value index,
@@ -83,6 +85,13 @@ constexpr int fast_classes(int n) {
   return n >= 192 && n % 8 == 0 ? 8 : (n % 4 == 0 ? 4 : (n % 2 == 0 ? 2 : 1));
 }
 
+// Longest line of the matrix kernels (dft_kernels.hpp), which serve every length
+// up to it, with or without fixed-length kernels. FP64 pairs at lengths without
+// fixed-length kernels, generic against matrix kernels: 143^3 136 / 101 us, 187^3
+// 842 / 205, 254^3 10317 / 796, 306^3 3833 / 1497, 343^3 1661 / 2765, 405^3 3462 /
+// 5019: past 306 the 7-smooth lengths run faster on the generic FFT.
+constexpr int kDftMaxLength = 320;
+
 // Geometry of the z kernels' LDS tile: sticks per workgroup, padded line
 // length and the padding shift of the index map i -> i + (i >> shift).
 template <typename T>
@@ -96,8 +105,8 @@ inline int fast_pitch(int nst) {
   return (nst + 1 + q - 1) / q * q;
 }
 
-// True when (nx, ny, nz) have fast kernels: z kernels and the split plane
-// stage for every length in {32, 36, 40, 42, 44, 45, 48, 50, 52, 54, 56, 60,
+// True when n is a fixed length: z kernels and the split plane stage for every
+// n in {32, 36, 40, 42, 44, 45, 48, 50, 52, 54, 56, 60,
 // 63, 64, 66, 70, 72, 75, 78, 80, 81, 84, 88, 90, 96, 98, 99, 100, 104, 105,
 // 108, 110, 112, 117, 120, 121, 125, 126, 128, 130, 132, 135, 140, 144, 147,
 // 150, 154, 156, 160, 162, 165, 168, 169, 175, 176, 180, 182, 189, 192, 195,
@@ -105,8 +114,9 @@ inline int fast_pitch(int nst) {
 // 256, 260, 264, 270, 273, 275, 280, 286, 288, 297, 300, 312, 320, 325, 330,
 // 336, 338, 351, 352, 360, 384, 390, 400, 416, 420, 432, 440, 448, 450, 462,
 // 480, 500, 512} (108 lengths).
-template <typename T>
-bool fast_path_supported(int nx, int ny, int nz, int ncol, bool r2c);
+bool fixed_length(int n);
+// True when z transforms of length n have kernels here (fixed or matrix).
+inline bool z_supported(int n) { return fixed_length(n) || n <= kDftMaxLength; }
 // True when the class-split plane kernels serve the plane too: nx = ny in
 // {32, 64, 96, 128, 192} and their LDS fits ncol columns.
 template <typename T>

@@ -24,12 +24,12 @@ struct TuneState {
   std::map<std::string, TuneChoice> choices;
   std::map<int, std::string> arch;  // device -> "gfx950:256"
   // choices this process has used, by numeric key
-  std::map<std::tuple<int, int, int, int, int, int, int, int, int>, TuneChoice> used;
+  std::map<std::tuple<int, int, int, int, int, int, int, int, int, int>, TuneChoice> used;
 };
 
-std::tuple<int, int, int, int, int, int, int, int, int> numeric(const TuneKey& k) {
+std::tuple<int, int, int, int, int, int, int, int, int, int> numeric(const TuneKey& k) {
   return std::make_tuple(k.device, k.valueBytes, k.n, k.ny, k.nz, k.r2c, k.forward, k.ncolBucket,
-                         k.countBucket);
+                         k.stickBucket, k.countBucket);
 }
 
 TuneState& state() {
@@ -51,7 +51,7 @@ std::string cache_path() {
   } else {
     return std::string();
   }
-  return base + "/spfft_amd/tune-v1.txt";
+  return base + "/spfft_amd/tune-v2.txt";
 }
 
 // mkdir -p of the directory part of `path`
@@ -78,7 +78,7 @@ void load_locked(TuneState& s) {
     TuneChoice c;
     if (std::sscanf(line, "%255s plane=%d slots=%d zruns=%d", key, &c.plane, &c.slots,
                     &c.zRuns) == 4 &&
-        c.plane >= 0 && c.plane <= 2 && c.slots >= 0 && c.slots <= 64 &&
+        c.plane >= 0 && c.plane <= 3 && c.slots >= 0 && c.slots <= 64 &&
         (c.zRuns == 0 || c.zRuns == 1)) {
       s.choices[key] = c;
     }
@@ -93,7 +93,7 @@ void save_locked(const TuneState& s) {
   FILE* f = std::fopen(tmp.c_str(), "w");
   if (!f) return;
   std::fprintf(f, "# spfft_amd kernel choices: <arch:CUs:bytes:N[xNy]:Nz:type:direction:"
-                  "columns:transforms> plane= slots= zruns=\n");
+                  "columns:sticks:transforms> plane= slots= zruns=\n");
   for (const auto& kv : s.choices) {
     std::fprintf(f, "%s plane=%d slots=%d zruns=%d\n", kv.first.c_str(), kv.second.plane,
                  kv.second.slots, kv.second.zRuns);
@@ -108,10 +108,17 @@ int round_pow2(int v) {
   return p;
 }
 
+// v rounded up to 4, 5, 6 or 7 times a power of two.
+int round_quarter(int v) {
+  int step = 1;
+  while (v > 8 * step) step *= 2;
+  return (v + step - 1) / step * step;
+}
+
 }  // namespace
 
 TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2c, bool forward,
-                      int maxNcol, int count) {
+                      int maxNcol, int maxNst, int count) {
   TuneKey k;
   k.device = device;
   k.valueBytes = valueBytes;
@@ -121,6 +128,7 @@ TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2
   k.r2c = r2c ? 1 : 0;
   k.forward = forward ? 1 : 0;
   k.ncolBucket = (maxNcol + 15) / 16 * 16;
+  k.stickBucket = round_quarter(maxNst);
   k.countBucket = round_pow2(count < 1 ? 1 : count);
   return k;
 }
@@ -152,7 +160,7 @@ std::string tune_key_text(const TuneKey& k) {
   if (k.ny != k.n) o << "x" << k.ny;
   o << ":Z" << k.nz << ":"
     << (k.r2c ? "r2c" : "c2c") << ":" << (k.forward ? "fwd" : "bwd") << ":col" << k.ncolBucket
-    << ":x" << k.countBucket;
+    << ":st" << k.stickBucket << ":x" << k.countBucket;
   return o.str();
 }
 
