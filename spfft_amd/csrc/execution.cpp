@@ -146,26 +146,20 @@ struct TuneEvents {
   TuneEvents& operator=(const TuneEvents&) = delete;
 };
 
-// SPFFT_AMD_GRAPHS=0 replays batched calls with direct launches instead of
-// captured HIP graphs.
-bool graphs_enabled() {
-  const char* v = std::getenv("SPFFT_AMD_GRAPHS");
-  return !(v && v[0] == '0');
-}
-
 std::atomic<std::uint64_t> next_serial{1};
 
-// A batched call's device argument table, block map and captured launch
-// chain, keyed by everything they depend on: direction, device, and per
-// transform its serial number (never reused, so a destroyed transform's plan
-// can never match again), its device input/output pointers and scaling.
+// A batched call's device argument table and block map, keyed by everything they
+// hold: direction, device, and per transform its serial number (never reused, so
+// a destroyed transform's plan can never match again), its device input/output
+// pointers and scaling. The launches are issued directly: a captured graph of the
+// two or three of them took 30 to 40 us of host time to replay against 15 for the
+// launches, and 300 us to make.
 struct BatchPlan {
   std::vector<std::uint64_t> key;
+  int device = 0;
   void* args = nullptr;
   void* map = nullptr;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
-  TuneChoice choice;  // kernel choices the graph was captured with
+  size_t argBytes = 0, mapBytes = 0;
 };
 
 // Most recently used first. Heap-allocated and never destroyed: plans hold
@@ -181,12 +175,16 @@ BatchCache& batch_cache() {
   return *cache;
 }
 
-void release_plan(BatchPlan& p) {
-  if (p.exec) (void)hipGraphExecDestroy(p.exec);
-  if (p.graph) (void)hipGraphDestroy(p.graph);
-  if (p.args) (void)hipFree(p.args);
-  if (p.map) (void)hipFree(p.map);
-  p = BatchPlan{};
+// Device memory of at least `bytes`, kept when it is large enough. Work queued
+// on the default stream may still read the old contents: they are replaced on
+// that stream.
+void grow(void** ptr, size_t* have, size_t bytes) {
+  if (*have >= bytes) return;
+  if (*ptr) check_hip(hipFree(*ptr));  // waits for the device
+  *ptr = nullptr;
+  *have = 0;
+  check_hip(hipMalloc(ptr, bytes));
+  *have = bytes;
 }
 
 }  // namespace
@@ -990,8 +988,10 @@ void ExecutionGPU<T>::fill_batch_tables(ExecutionGPU<T>* const* ex, size_t n, co
     f.out = dout[t];
     f.useScale = forward && scaling[t] == SPFFT_FULL_SCALING ? 1 : 0;
     f.pitchA = ex[t]->classSplit_ ? fast_xy_pitch_a<T>(ex[0]->map_->dimX, f.ncol) : 0;
-    const int b = (f.nst + S - 1) / S;
-    for (int j = 0; j < b; ++j) zmap[k++] = make_int2(static_cast<int>(t), j);
+    if (zmap) {
+      const int b = (f.nst + S - 1) / S;
+      for (int j = 0; j < b; ++j) zmap[k++] = make_int2(static_cast<int>(t), j);
+    }
     args[t] = f;
   }
 }
@@ -1159,25 +1159,34 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   auto hit = std::find_if(cache.plans.begin(), cache.plans.end(),
                           [&](const BatchPlan& p) { return p.key == key; });
   if (hit == cache.plans.end()) {
-    if (cache.plans.size() >= kMaxBatchPlans) {
-      // the evicted plan's tables may still be read by queued work
-      check_hip(hipStreamSynchronize(nullptr));
-      release_plan(cache.plans.back());
-      cache.plans.pop_back();
+    if (cache.plans.size() < kMaxBatchPlans) {
+      cache.plans.emplace_front();
+    } else {
+      // the least recently used plan on this device gives its memory, else the
+      // least recently used one
+      hit = std::prev(cache.plans.end());
+      for (auto p = cache.plans.begin(); p != cache.plans.end(); ++p) {
+        if (p->device == shape.device) hit = p;
+      }
+      cache.plans.splice(cache.plans.begin(), cache.plans, hit);
+    }
+    BatchPlan& plan = cache.plans.front();
+    plan.key.clear();  // holds nothing until the tables are on their way
+    if (plan.device != shape.device) {
+      if (plan.args) check_hip(hipFree(std::exchange(plan.args, nullptr)));
+      if (plan.map) check_hip(hipFree(std::exchange(plan.map, nullptr)));
+      plan.argBytes = plan.mapBytes = 0;
+      plan.device = shape.device;
     }
     std::vector<FastArgs<T>> args(n);
-    std::vector<int2> zmap(shape.blocks);
     fill_batch_tables(ex.data(), n, din.data(), dout.data(), forward,
-                      forward ? scaling.data() : nullptr, args.data(), zmap.data());
-    BatchPlan plan;
+                      forward ? scaling.data() : nullptr, args.data(), nullptr);
+    grow(&plan.args, &plan.argBytes, n * sizeof(FastArgs<T>));
+    grow(&plan.map, &plan.mapBytes, static_cast<size_t>(shape.blocks) * sizeof(int2));
+    launch_batch_tables<T>(args.data(), nt, sticks_per_block<T>(shape.dimZ),
+                           static_cast<FastArgs<T>*>(plan.args), static_cast<int2*>(plan.map),
+                           nullptr);
     plan.key = std::move(key);
-    check_hip(hipMalloc(&plan.args, n * sizeof(FastArgs<T>)));
-    check_hip(hipMalloc(&plan.map, zmap.size() * sizeof(int2)));
-    check_hip(hipMemcpyAsync(plan.args, args.data(), n * sizeof(FastArgs<T>),
-                             hipMemcpyHostToDevice, nullptr));
-    check_hip(hipMemcpyAsync(plan.map, zmap.data(), zmap.size() * sizeof(int2),
-                             hipMemcpyHostToDevice, nullptr));
-    cache.plans.push_front(std::move(plan));
     hit = cache.plans.begin();
   } else if (hit != cache.plans.begin()) {
     cache.plans.splice(cache.plans.begin(), cache.plans, hit);
@@ -1211,38 +1220,7 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   if (choice.plane != 1) {
     choice.plane = served_plane(choice.plane, shape.classSplit, shape.split, shape.matrix);
   }
-  if (plan.exec && (plan.choice.plane != choice.plane || plan.choice.slots != choice.slots ||
-                    plan.choice.zRuns != choice.zRuns)) {
-    (void)hipGraphExecDestroy(plan.exec);
-    (void)hipGraphDestroy(plan.graph);
-    plan.exec = nullptr;
-    plan.graph = nullptr;
-  }
-  if (!graphs_enabled() || prof::enabled()) {
-    launch_batch(forward, shape, nt, choice, dArgs, dMap, nullptr);
-    return true;
-  }
-  if (!plan.exec) {
-    plan.choice = choice;
-    // Capture the two launches once on a private stream; later calls with
-    // the same key replay the graph on the default stream.
-    hipStream_t cs = nullptr;
-    check_hip(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-    check_hip(hipStreamBeginCapture(cs, hipStreamCaptureModeRelaxed));
-    try {
-      launch_batch(forward, shape, nt, choice, dArgs, dMap, cs);
-    } catch (...) {
-      hipGraph_t g = nullptr;
-      (void)hipStreamEndCapture(cs, &g);
-      if (g) (void)hipGraphDestroy(g);
-      (void)hipStreamDestroy(cs);
-      throw;
-    }
-    check_hip(hipStreamEndCapture(cs, &plan.graph));
-    check_hip(hipStreamDestroy(cs));
-    check_hip(hipGraphInstantiate(&plan.exec, plan.graph, nullptr, nullptr, 0));
-  }
-  check_hip(hipGraphLaunch(plan.exec, nullptr));
+  launch_batch(forward, shape, nt, choice, dArgs, dMap, nullptr);
   return true;
 }
 

@@ -68,13 +68,12 @@ public:
   // additionally makes the default stream wait for its stream.
   void synchronize(SpfftExecType mode, bool concurrent = false);
 
-  // Batched execution of several transforms of one shape on the fixed-length
-  // or matrix kernels: one z launch and one xy launch (two for the split stage)
-  // for the whole batch, on the default stream. The argument tables and the captured launch chain (a HIP graph)
-  // are kept for the most recent batches and replayed when the same
-  // transforms are called again with the same pointers. Returns false without
-  // doing anything when the batch does not qualify (different shapes,
-  // generic lengths, host pointers, empty sets).
+  // Batched execution of several transforms of one shape on the fixed-length or
+  // matrix kernels: one z launch and one xy launch (two for the split stage) for
+  // the whole batch, on the default stream. The argument tables are kept for the
+  // most recent batches and read again when the same transforms are called with
+  // the same pointers. Returns false without doing anything when the batch does
+  // not qualify (different shapes, generic lengths, host pointers, empty sets).
   static bool run_batch(const std::vector<ExecutionGPU<T>*>& ex, const std::vector<const T*>& in,
                         const std::vector<T*>& out, bool forward,
                         const std::vector<SpfftScalingType>& scaling);
@@ -102,7 +101,8 @@ public:
   static bool plane_candidate(ExecutionGPU* const* ex, size_t n, const T* const* din,
                               T* const* dout, bool forward, const BatchShape& shape);
   // Host copies of the argument table (n entries) and the z block map
-  // (shape.blocks entries); `scaling` is read for forward batches only.
+  // (shape.blocks entries, none if null); `scaling` is read for forward batches
+  // only.
   static void fill_batch_tables(ExecutionGPU* const* ex, size_t n, const T* const* din,
                                 T* const* dout, bool forward, const SpfftScalingType* scaling,
                                 FastArgs<T>* args, int2* zmap);

@@ -137,6 +137,13 @@ template <typename T>
 void launch_fast_xy_batch(bool forward, bool r2c, int n, const FastArgs<T>* batch, int ntrans,
                           int nz, int maxNcol, hipStream_t stream);
 
+// Writes a batch's argument table and its z block map, (transform, block) for
+// every `sticks` sticks of every transform, from kernel arguments: ordered on
+// `stream` like any launch, with no host buffer to keep.
+template <typename T>
+void launch_batch_tables(const FastArgs<T>* host, int ntrans, int sticks, FastArgs<T>* args,
+                         int2* map, hipStream_t stream);
+
 // Whole-plane kernels for batches (one workgroup per plane; no class split,
 // so the plane's input is read once): power-of-two lengths up to 128, C2C,
 // when the plane tile for `ncol` columns fits in LDS.

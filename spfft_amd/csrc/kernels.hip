@@ -13,6 +13,7 @@
 #include <mutex>
 #include <unordered_map>
 
+#include "fast_kernels.hpp"
 #include "hip_check.hpp"
 #include "kernels.hpp"
 #include "profiling.hpp"
@@ -391,6 +392,32 @@ __global__ void k_twiddles(Tw<T>* tw, int n) {
   }
 }
 
+// One launch's share of a batch's tables (see launch_batch_tables): as many
+// transforms as the 4 KiB of kernel arguments hold. Workgroup t writes entry t
+// of the argument table and its transform's part of the block map.
+constexpr int kTableTransforms = 12;
+template <typename T>
+struct TableShare {
+  FastArgs<T> a[kTableTransforms];
+  int block0[kTableTransforms];  // first map entry
+  int first = 0, sticks = 1;
+};
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    k_batch_tables(TableShare<T> s, FastArgs<T>* args, int2* map) {
+  static_assert(sizeof(FastArgs<T>) % 4 == 0 && sizeof(FastArgs<T>) / 4 <= kBlock,
+                "one dword per thread");
+  static_assert(sizeof(s) <= 4000, "kernel arguments");
+  const int t = blockIdx.x;
+  const unsigned* from = reinterpret_cast<const unsigned*>(&s.a[t]);
+  unsigned* to = reinterpret_cast<unsigned*>(args + s.first + t);
+  if (threadIdx.x < sizeof(FastArgs<T>) / 4) to[threadIdx.x] = from[threadIdx.x];
+  const int blocks = (s.a[t].nst + s.sticks - 1) / s.sticks;
+  for (int j = threadIdx.x; j < blocks; j += kBlock) {
+    map[s.block0[t] + j] = make_int2(s.first + t, j);
+  }
+}
+
 // Raise the dynamic LDS limit of a kernel once per process.
 template <typename Kernel>
 void launch_stage(Kernel kernel, dim3 grid, size_t lds, hipStream_t stream,
@@ -451,6 +478,25 @@ void generate_twiddles(Tw<T>* tw, int n, hipStream_t stream) {
   check_launch();
 }
 
+template <typename T>
+void launch_batch_tables(const FastArgs<T>* host, int ntrans, int sticks, FastArgs<T>* args,
+                         int2* map, hipStream_t stream) {
+  int blocks = 0;
+  for (int t0 = 0; t0 < ntrans; t0 += kTableTransforms) {
+    TableShare<T> s;
+    const int n = std::min(kTableTransforms, ntrans - t0);
+    s.first = t0;
+    s.sticks = sticks;
+    for (int t = 0; t < n; ++t) {
+      s.a[t] = host[t0 + t];
+      s.block0[t] = blocks;
+      blocks += (host[t0 + t].nst + sticks - 1) / sticks;
+    }
+    hipLaunchKernelGGL(k_batch_tables<T>, dim3(n), dim3(kBlock), 0, stream, s, args, map);
+    check_launch();
+  }
+}
+
 #define SPFFT_STAGE_LAUNCHER(NAME, KERNEL, LEN, COUNT, GRID)                      \
   template <typename T>                                                          \
   void NAME(const StageArgs<T>& a, hipStream_t stream) {                         \
@@ -481,6 +527,8 @@ SPFFT_STAGE_LAUNCHER(launch_z_forward, k_z_forward, nz, a.nst,
 #define SPFFT_INSTANTIATE(T)                                                      \
   template int stage_batch<T>(int, int, size_t*);                                \
   template void generate_twiddles<T>(Tw<T>*, int, hipStream_t);                  \
+  template void launch_batch_tables<T>(const FastArgs<T>*, int, int, FastArgs<T>*, int2*, \
+                                       hipStream_t);                             \
   template void launch_z_backward<T>(const StageArgs<T>&, hipStream_t);          \
   template void launch_y_backward<T>(const StageArgs<T>&, hipStream_t);          \
   template void launch_x_backward<T>(const StageArgs<T>&, hipStream_t);          \
