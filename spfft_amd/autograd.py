@@ -28,9 +28,19 @@ first waits for it and the current stream then waits for the transform.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 import spfft_amd as sp
+
+_i, _ll, _vp = ctypes.c_int, ctypes.c_longlong, ctypes.c_void_p
+sp.lib.spfft_amd_energy_partials.argtypes = [_i]
+sp.lib.spfft_amd_energy_partials.restype = _i
+sp.lib.spfft_amd_field_energy.argtypes = [_i, _vp, _vp, _ll, _i, _vp, _vp, _vp]
+sp.lib.spfft_amd_field_energy.restype = _i
+sp.lib.spfft_amd_energy_field.argtypes = [_i, _vp, _vp, _vp, _ll, _i, _vp, _vp]
+sp.lib.spfft_amd_energy_field.restype = _i
 
 
 def _dtype(transform):
@@ -148,6 +158,13 @@ def _field_budget(memory_budget):
     return free // 4
 
 
+def _rows(x):
+    """Addresses of x[0], x[1], ... of a contiguous complex tensor."""
+    x = torch.view_as_real(x)  # refuses a lazily conjugated one
+    step = x[0].numel() * x.element_size()
+    return [x.data_ptr() + b * step for b in range(x.shape[0])]
+
+
 def _batch_backward(transforms, dims, C):
     nx, ny, nz = dims
     n = transforms[0].num_values
@@ -161,10 +178,7 @@ def _batch_backward(transforms, dims, C):
     C = C.contiguous()
     psi = torch.empty((len(transforms), nz, ny, nx), dtype=C.dtype, device=C.device)
     with _OnDefaultStream():
-        sp.multi_transform_backward(transforms, [torch.view_as_real(C[b]).data_ptr()
-                                                 for b in range(len(transforms))],
-                                    [torch.view_as_real(psi[b]).data_ptr()
-                                     for b in range(len(transforms))])
+        sp.multi_transform_backward(transforms, _rows(C), _rows(psi))
     return psi
 
 
@@ -172,10 +186,7 @@ def _batch_adjoint(transforms, n, fields):
     out = torch.empty((len(transforms), n), dtype=fields.dtype, device=fields.device)
     fields = fields.contiguous()
     with _OnDefaultStream():
-        sp.multi_transform_forward(transforms, [torch.view_as_real(fields[b]).data_ptr()
-                                                for b in range(len(transforms))],
-                                   [torch.view_as_real(out[b]).data_ptr()
-                                    for b in range(len(transforms))],
+        sp.multi_transform_forward(transforms, _rows(fields), _rows(out),
                                    [sp.SPFFT_NO_SCALING] * len(transforms))
     return out
 
@@ -190,12 +201,59 @@ def recompute_fields(field_bytes, recompute="auto", memory_budget=None):
     return bool(recompute)
 
 
+def _fused(psi, potential):
+    """The energy kernels take a potential that is one contiguous field of the
+    bands' real type on their device; any other goes through tensor expressions."""
+    real = torch.float64 if psi.dtype == torch.complex128 else torch.float32
+    return (potential.device == psi.device and potential.dtype == real and
+            potential.shape == psi.shape[1:] and potential.is_contiguous() and
+            not potential.is_neg() and psi.is_contiguous() and not psi.is_conj() and
+            psi.shape[0] <= 65535)
+
+
+def _band_energy(psi, potential):
+    """sum_b sum_r V |psi_b|^2 in float64."""
+    if not _fused(psi, potential):
+        return torch.sum(potential.to(torch.float64) *
+                         torch.sum((psi.real ** 2 + psi.imag ** 2).to(torch.float64), dim=0))
+    bands = psi.shape[0]
+    partial = torch.empty(sp.lib.spfft_amd_energy_partials(bands), dtype=torch.float64,
+                          device=psi.device)
+    energy = torch.empty((), dtype=torch.float64, device=psi.device)
+    sp._check(sp.lib.spfft_amd_field_energy(
+        potential.element_size(), psi.data_ptr(), potential.data_ptr(), potential.numel(), bands,
+        partial.data_ptr(), energy.data_ptr(), torch.cuda.current_stream().cuda_stream),
+        "field_energy")
+    return energy
+
+
+def _energy_gradient(transforms, psi, own, potential, grad_energy):
+    """grad_energy * 2 B^H (V psi) per band. own: psi belongs to the call, so the
+    field may take its place."""
+    n = transforms[0].num_values
+    # a gradient that is itself differentiated stays a tensor expression
+    if not _fused(psi, potential) or (torch.is_grad_enabled() and grad_energy.requires_grad):
+        g = _batch_adjoint(transforms, n, (2.0 * potential) * psi)
+        return grad_energy.to(potential.dtype) * g
+    # FP64: the factor goes into the field; FP32: its product with the potential
+    # could leave float32's range where the gradient does not
+    scale = (grad_energy if potential.dtype == torch.float64 and
+             grad_energy.dtype == torch.float64 and grad_energy.device == psi.device and
+             not grad_energy.is_neg() else None)
+    field = psi if own else torch.empty_like(psi)
+    sp._check(sp.lib.spfft_amd_energy_field(
+        potential.element_size(), psi.data_ptr(), potential.data_ptr(),
+        None if scale is None else scale.data_ptr(), potential.numel(), psi.shape[0],
+        field.data_ptr(), torch.cuda.current_stream().cuda_stream), "energy_field")
+    g = _batch_adjoint(transforms, n, field)
+    return g if scale is not None else grad_energy.to(potential.dtype) * g
+
+
 class SparseEnergyBatch(torch.autograd.Function):
     @staticmethod
     def forward(ctx, C, potential, transforms, dims, recompute="auto", memory_budget=None):
         psi = _batch_backward(transforms, dims, C)
-        energy = torch.sum(potential.to(torch.float64) *
-                           torch.sum((psi.real ** 2 + psi.imag ** 2).to(torch.float64), dim=0))
+        energy = _band_energy(psi, potential)
         ctx.transforms, ctx.dims = transforms, dims
         ctx.recompute = recompute_fields(psi.numel() * psi.element_size(), recompute,
                                          memory_budget)
@@ -211,9 +269,9 @@ class SparseEnergyBatch(torch.autograd.Function):
             C, potential = ctx.saved_tensors
             psi = _batch_backward(ctx.transforms, ctx.dims, C)
         else:
-            C, potential, psi = ctx.saved_tensors
-        g = _batch_adjoint(ctx.transforms, C.shape[1], (2.0 * potential) * psi)
-        return grad_energy.to(potential.dtype) * g, None, None, None, None, None
+            _, potential, psi = ctx.saved_tensors
+        g = _energy_gradient(ctx.transforms, psi, ctx.recompute, potential, grad_energy)
+        return g, None, None, None, None, None
 
 
 def sparse_energy_batch(C, potential, transforms, dims, recompute="auto", memory_budget=None):
