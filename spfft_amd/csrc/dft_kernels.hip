@@ -616,7 +616,7 @@ __device__ __forceinline__ void z_forward_dft(const FastArgs<T>& a, int trigAt, 
 // 8 of its transform): workgroups are dealt to the 8 XCDs round robin, so the
 // parts of a plane share one XCD's L2 for the plane's input.
 struct PlaneArgs {
-  int nx, ny;
+  int nx, ny, nz;
   int slotShift;     // log2 of the slots per workgroup
   int even;          // forward: parts of even output indices
   int blocks;        // plane blocks of a transform (batches)
@@ -632,16 +632,88 @@ __host__ __device__ constexpr int tile_pitch(int ny, int ky, int rows, bool stag
   return (in > out ? in : out) | 1;
 }
 
+template <typename T>
+__device__ __forceinline__ Trig trig_of(Tw<T> w) {
+  if constexpr (sizeof(T) == 4) {
+    return Trig{static_cast<double>(w.hi.re) + static_cast<double>(w.lo.re),
+                -(static_cast<double>(w.hi.im) + static_cast<double>(w.lo.im))};
+  } else {
+    return Trig{w.re, -w.im};
+  }
+}
+__device__ __forceinline__ Cd rotated(Cd acc, Cd x, Trig t) {  // acc + x exp(i t)
+  return Cd{fma(x.re, t.c, fma(-x.im, t.s, acc.re)), fma(x.re, t.s, fma(x.im, t.c, acc.im))};
+}
+// Every stick's z sum at plane z into its tile cell: four lanes per stick, whose
+// values are one run (FastArgs::zInfo).
+template <typename T, bool RC>
+__device__ __forceinline__ void sum_values(const FastArgs<T>& a, int n, int z, const Trig* tab,
+                                           int P, Cx<T>* Y) {
+  constexpr int L = 4, U = 4;
+  const Cx<T>* in = reinterpret_cast<const Cx<T>*>(a.in);
+  const int sub = threadIdx.x % L, step = blockDim.x / L;
+  const int inc = L * z % n;
+#pragma unroll 1
+  for (int s = threadIdx.x / L; s < a.nst; s += step) {
+    const int4 run = a.zInfo[s];
+    const int cell = a.stickCell[s];
+    Cd acc = Cd{0.0, 0.0};
+    if (RC && s == 0 && a.zeroZeroStick == 0) {
+      // the (0,0) stick is filled hermitian, pair by pair
+      auto value = [&](int i) {
+        int pos = i - run.y;
+        pos += pos < 0 ? n : 0;
+        return pos < run.z ? in[run.x + pos] : Cx<T>{T(0), T(0)};
+      };
+      for (int r = sub; r <= a.kz; r += L) {
+        Pair<T> x;
+        x.p = value(r);
+        x.m = r != 0 && 2 * r != n ? value(n - r) : Cx<T>{T(0), T(0)};
+        x = hermitian_pair(x, n, r);
+        Trig t = tab[r * z % n];
+        acc = rotated(acc, wide(x.p), t);
+        t.s = -t.s;
+        acc = rotated(acc, wide(x.m), t);
+      }
+    } else {
+      int idx = (run.y + sub) * z % n;
+#pragma unroll 1
+      for (int p0 = sub; p0 < run.z; p0 += U * L) {
+        Cx<T> x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = in[run.x + min(p0 + u * L, run.z - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (p0 + u * L < run.z) acc = rotated(acc, wide(x[u]), tab[idx]);
+          idx += inc;
+          idx -= idx >= n ? n : 0;
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 1; d < L; d *= 2) {
+      acc.re += __shfl_xor(acc.re, d);
+      acc.im += __shfl_xor(acc.im, d);
+    }
+    if (sub == 0) Y[(cell >> 16) * P + (cell & 0xffff)] = narrow<T>(acc.re, acc.im);
+  }
+}
+
+// How the sticks of a plane reach the backward kernel: gathered from the [z]
+// [stick] buffer through the [column][y] table (no room in LDS for more), from
+// one pass over the plane's stick row into the tile as [column][folded y], or
+// summed over z from the values themselves, with no z kernel before.
+enum Source { kGather, kStaged, kValues };
+
 // Backward: a workgroup owns the rows of its output slots of y. It computes
 // those rows of every column, keeps them in LDS as [column][row], and transforms
-// the rows. STAGED: the plane's sticks enter through the tile as [column][folded
-// y], read in one pass over the plane's stick row; a wave's 16 columns are its
-// own, so their rows overwrite them. Else (no room in LDS) the sticks are
-// gathered from the row through the [column][y] table.
-template <typename T, bool RC, bool EX, bool EY, bool STAGED>
+// the rows. A wave's 16 columns are its own, so their rows overwrite their
+// sticks.
+template <typename T, bool RC, bool EX, bool EY, Source SRC>
 __device__ __forceinline__ void xy_backward_dft(const FastArgs<T>& a, const PlaneArgs& p, int z,
                                                 int part) {
   if (z >= a.nz) return;
+  constexpr bool STAGED = SRC != kGather;
   const int nx = p.nx, ny = p.ny;
   constexpr int TY = EY ? 4 : 2, TX = EX ? 4 : 2;
   const int S = 1 << p.slotShift, rows = TY * S;
@@ -664,7 +736,14 @@ __device__ __forceinline__ void xy_backward_dft(const FastArgs<T>& a, const Plan
   using Sums = OutSums<T, EY, true, false, EY ? 1 : 2, !STAGED>;
   typename Sums::Roots head;
   head.first(ny, ky, q0, trig + p.trigY);  // every tile's: one tile of slots
-  if (STAGED) {
+  if constexpr (SRC == kValues) {
+    const int nz = p.nz;
+    Trig* tabZ = reinterpret_cast<Trig*>(Y + cols * P);
+    for (int t = threadIdx.x; t < nz; t += threads) tabZ[t] = trig_of<T>(a.twZ[t]);
+    for (int t = threadIdx.x; t < cols * P; t += threads) Y[t] = Cx<T>{T(0), T(0)};
+    lds_barrier();
+    sum_values<T, RC>(a, nz, z, tabZ, P, Y);
+  } else if constexpr (STAGED) {
     // stickCell: tile column << 16 | folded y
     constexpr int U = 4;
     Cx<T> x[U];
@@ -895,14 +974,14 @@ __global__ void __launch_bounds__(kZWaves * kWave)
   a.hasRuns = a.hasRuns && useRuns;
   z_forward_dft<T, EVEN>(a, trigAt, m.y);
 }
-// STAGED: backward only
-template <typename T, bool FWD, bool RC, bool EX, bool EY, bool STAGED>
+// SRC: backward only
+template <typename T, bool FWD, bool RC, bool EX, bool EY, Source SRC>
 __device__ __forceinline__ void xy_dft(const FastArgs<T>& a, const PlaneArgs& p, int block) {
   const int z = a.zBegin + 8 * block + static_cast<int>(blockIdx.x);
   if constexpr (FWD) {
     xy_forward_dft<T, RC, EX, EY>(a, p, z, blockIdx.y);
   } else {
-    xy_backward_dft<T, RC, EX, EY, STAGED>(a, p, z, blockIdx.y);
+    xy_backward_dft<T, RC, EX, EY, SRC>(a, p, z, blockIdx.y);
   }
 }
 // Waves per SIMD: two workgroups of eight waves share a CU where the kernel's
@@ -911,16 +990,16 @@ template <bool FWD, bool EX, bool EY>
 constexpr int plane_waves() {
   return !FWD && (EX || EY) ? 3 : 4;
 }
-template <typename T, bool FWD, bool RC, bool EX, bool EY, bool STAGED>
+template <typename T, bool FWD, bool RC, bool EX, bool EY, Source SRC>
 __global__ void __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(plane_waves<FWD, EX, EY>())))
     k_xy_dft(FastArgs<T> a, PlaneArgs p) {
-  xy_dft<T, FWD, RC, EX, EY, STAGED>(a, p, blockIdx.z);
+  xy_dft<T, FWD, RC, EX, EY, SRC>(a, p, blockIdx.z);
 }
-template <typename T, bool FWD, bool RC, bool EX, bool EY, bool STAGED>
+template <typename T, bool FWD, bool RC, bool EX, bool EY, Source SRC>
 __global__ void __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(plane_waves<FWD, EX, EY>())))
     k_xy_dft_batch(const FastArgs<T>* __restrict__ batch, PlaneArgs p) {
   const int t = blockIdx.z / p.blocks;
-  xy_dft<T, FWD, RC, EX, EY, STAGED>(on_global(batch[t], batch), p, blockIdx.z - t * p.blocks);
+  xy_dft<T, FWD, RC, EX, EY, SRC>(on_global(batch[t], batch), p, blockIdx.z - t * p.blocks);
 }
 
 // Raise the dynamic LDS limit of a kernel once per process.
@@ -955,7 +1034,7 @@ struct Plan {
   int slotShift = 0;    // log2 of the slots per workgroup
   int even = 0;         // forward: workgroups of even output indices (even lengths)
   int waves = 4;        // per workgroup
-  bool staged = false;  // backward: sticks through the tile
+  Source source = kGather;  // backward
   size_t lds = 0;
 };
 
@@ -963,9 +1042,9 @@ struct Plan {
 // it. A part costs a whole tile of 16 slots in its first transform however few
 // it owns, so a plane is cut into fewer slots per part only while the launch
 // leaves most CUs idle or the tile does not fit in LDS, and never below one tile
-// of 16 rows (columns).
+// of 16 rows (columns). nz > 0: backward from the values.
 template <typename T>
-Plan plane_plan(bool forward, bool r2c, int nx, int ny, int kx, int ky, int planes) {
+Plan plane_plan(bool forward, bool r2c, int nx, int ny, int kx, int ky, int planes, int nz = 0) {
   constexpr int kEnough = 160;  // workgroups, of 256 CUs
   Plan plan;
   const bool evenX = nx % 2 == 0;
@@ -983,8 +1062,9 @@ Plan plane_plan(bool forward, bool r2c, int nx, int ny, int kx, int ky, int plan
         return 4 * kTile * sizeof(int) + static_cast<size_t>(tile_columns(nx, kx, r2c)) *
                                              tile_pitch(ny, ky, lines, staged) * sizeof(Cx<T>);
       };
-      plan.staged = bytes(true) <= kLdsMax;
-      plan.lds = bytes(plan.staged);
+      plan.source = bytes(true) <= kLdsMax ? kStaged : kGather;
+      if (nz > 0) plan.source = kValues;
+      plan.lds = bytes(plan.source != kGather) + nz * sizeof(Trig);
     }
     if (lines <= kTile) break;
     if (plan.lds <= kLdsMax && planes * plan.parts >= kEnough && slots / 2 < total) break;
@@ -995,45 +1075,48 @@ Plan plane_plan(bool forward, bool r2c, int nx, int ny, int kx, int ky, int plan
   const int work = forward ? std::max(tiles(ny), tiles(lines) * (tiles(ky + 1)))
                            : std::max(tile_columns(nx, kx, r2c) / kTile,
                                       tiles(lines) * tiles(out_slots(nx)));
-  plan.waves = work > 4 ? kMaxWaves : 4;
+  // (and all of them for the sums over z)
+  plan.waves = work > 4 || plan.source == kValues ? kMaxWaves : 4;
   return plan;
 }
 
 // f(kernel) with the plane kernel for the run-time choices.
-template <typename T, bool BATCH, bool FWD, bool RC, typename F>
-void plane_kernel(bool evenX, bool evenY, bool staged, F&& f) {
-#define SPFFT_PLANE_CASE(EX, EY, STAGED)                                \
-  if (evenX == EX && evenY == EY && (FWD || staged == STAGED)) {        \
-    if constexpr (BATCH) {                                              \
-      f(k_xy_dft_batch<T, FWD, RC, EX, EY, FWD || STAGED>);             \
-    } else {                                                            \
-      f(k_xy_dft<T, FWD, RC, EX, EY, FWD || STAGED>);                   \
-    }                                                                   \
-    return;                                                             \
+template <typename T, bool BATCH, bool FWD, bool RC, Source SRC, typename F>
+void plane_kernel(bool evenX, bool evenY, F&& f) {
+#define SPFFT_PLANE_CASE(EX, EY)                          \
+  if (evenX == EX && evenY == EY) {                       \
+    if constexpr (BATCH) {                                \
+      return f(k_xy_dft_batch<T, FWD, RC, EX, EY, SRC>);  \
+    } else {                                              \
+      return f(k_xy_dft<T, FWD, RC, EX, EY, SRC>);        \
+    }                                                     \
   }
-  SPFFT_PLANE_CASE(true, true, true)
-  SPFFT_PLANE_CASE(true, false, true)
-  SPFFT_PLANE_CASE(false, true, true)
-  SPFFT_PLANE_CASE(false, false, true)
-  SPFFT_PLANE_CASE(true, true, false)
-  SPFFT_PLANE_CASE(true, false, false)
-  SPFFT_PLANE_CASE(false, true, false)
-  SPFFT_PLANE_CASE(false, false, false)
+  SPFFT_PLANE_CASE(true, true)
+  SPFFT_PLANE_CASE(true, false)
+  SPFFT_PLANE_CASE(false, true)
+  SPFFT_PLANE_CASE(false, false)
 #undef SPFFT_PLANE_CASE
 }
-template <typename T, bool BATCH, typename F>
-void plane_kernel(bool forward, bool r2c, bool evenX, bool evenY, bool staged, F&& f) {
+template <typename T, bool BATCH, bool RC, typename F>
+void plane_kernel(bool forward, bool evenX, bool evenY, Source source, F&& f) {
   if (forward) {
-    r2c ? plane_kernel<T, BATCH, true, true>(evenX, evenY, staged, f)
-        : plane_kernel<T, BATCH, true, false>(evenX, evenY, staged, f);
+    plane_kernel<T, BATCH, true, RC, kGather>(evenX, evenY, f);
+  } else if (source == kGather) {
+    plane_kernel<T, BATCH, false, RC, kGather>(evenX, evenY, f);
+  } else if (source == kStaged) {
+    plane_kernel<T, BATCH, false, RC, kStaged>(evenX, evenY, f);
   } else {
-    r2c ? plane_kernel<T, BATCH, false, true>(evenX, evenY, staged, f)
-        : plane_kernel<T, BATCH, false, false>(evenX, evenY, staged, f);
+    plane_kernel<T, BATCH, false, RC, kValues>(evenX, evenY, f);
   }
 }
+template <typename T, bool BATCH, typename F>
+void plane_kernel(bool forward, bool r2c, bool evenX, bool evenY, Source source, F&& f) {
+  r2c ? plane_kernel<T, BATCH, true>(forward, evenX, evenY, source, f)
+      : plane_kernel<T, BATCH, false>(forward, evenX, evenY, source, f);
+}
 
-PlaneArgs plane_args(const Plan& plan, const DftTables& t, int nx, int ny, int blocks) {
-  return PlaneArgs{nx, ny, plan.slotShift, plan.even, blocks, t.at[0], t.at[1]};
+PlaneArgs plane_args(const Plan& plan, const DftTables& t, int nx, int ny, int nz, int blocks) {
+  return PlaneArgs{nx, ny, nz, plan.slotShift, plan.even, blocks, t.at[0], t.at[1]};
 }
 
 }  // namespace
@@ -1047,26 +1130,33 @@ bool dft_plane_supported(bool r2c, int nx, int ny, int kx, int ky) {
 }
 
 template <typename T>
-void launch_dft_xy(bool forward, int nx, int ny, const FastArgs<T>& a, hipStream_t stream) {
-  const int planes = a.nz - a.zBegin;
-  const Plan plan = plane_plan<T>(forward, a.r2c != 0, nx, ny, a.kx, a.ky, planes);
-  const int blocks = (planes + 7) / 8;
-  const PlaneArgs p = plane_args(plan, DftTables(nx, ny, 1), nx, ny, blocks);
-  plane_kernel<T, false>(forward, a.r2c != 0, nx % 2 == 0, ny % 2 == 0, plan.staged,
-                         [&](auto kernel) {
-                           launch(kernel, forward ? "k_xy_forward_dft" : "k_xy_backward_dft",
-                                  dim3(8, plan.parts, blocks), plan.waves * kWave, plan.lds,
-                                  stream, a, p);
-                         });
+bool dft_values_supported(bool r2c, int nx, int ny, int nz, int kx, int ky) {
+  // any planes: the largest tile is the one of most slots
+  return dft_plane_supported<T>(r2c, nx, ny, kx, ky) &&
+         plane_plan<T>(false, r2c, nx, ny, kx, ky, 1 << 20, nz).lds <= kLdsMax;
 }
 
 template <typename T>
-void launch_dft_xy_batch(bool forward, bool r2c, int nx, int ny, int kx, int ky,
+void launch_dft_xy(bool forward, int nx, int ny, int fromValues, const FastArgs<T>& a,
+                   hipStream_t stream) {
+  const bool rc = a.r2c != 0;
+  const int planes = a.nz - a.zBegin;
+  const Plan plan = plane_plan<T>(forward, rc, nx, ny, a.kx, a.ky, planes, fromValues);
+  const int blocks = (planes + 7) / 8;
+  const PlaneArgs p = plane_args(plan, DftTables(nx, ny, 1), nx, ny, fromValues, blocks);
+  plane_kernel<T, false>(forward, rc, nx % 2 == 0, ny % 2 == 0, plan.source, [&](auto kernel) {
+    launch(kernel, forward ? "k_xy_forward_dft" : "k_xy_backward_dft",
+           dim3(8, plan.parts, blocks), plan.waves * kWave, plan.lds, stream, a, p);
+  });
+}
+
+template <typename T>
+void launch_dft_xy_batch(bool forward, bool r2c, int nx, int ny, int fromValues, int kx, int ky,
                          const FastArgs<T>* batch, int ntrans, int nz, hipStream_t stream) {
-  const Plan plan = plane_plan<T>(forward, r2c, nx, ny, kx, ky, nz * ntrans);
+  const Plan plan = plane_plan<T>(forward, r2c, nx, ny, kx, ky, nz * ntrans, fromValues);
   const int blocks = (nz + 7) / 8;
-  const PlaneArgs p = plane_args(plan, DftTables(nx, ny, 1), nx, ny, blocks);
-  plane_kernel<T, true>(forward, r2c, nx % 2 == 0, ny % 2 == 0, plan.staged, [&](auto kernel) {
+  const PlaneArgs p = plane_args(plan, DftTables(nx, ny, 1), nx, ny, fromValues, blocks);
+  plane_kernel<T, true>(forward, r2c, nx % 2 == 0, ny % 2 == 0, plan.source, [&](auto kernel) {
     launch(kernel, forward ? "k_xy_forward_dft_batch" : "k_xy_backward_dft_batch",
            dim3(8, plan.parts, blocks * ntrans), plan.waves * kWave, plan.lds, stream, batch, p);
   });
@@ -1101,9 +1191,10 @@ void launch_dft_z_batch(bool forward, bool r2c, int nx, int ny, int nz, int kz,
 
 #define SPFFT_INSTANTIATE_DFT(T)                                                              \
   template bool dft_plane_supported<T>(bool, int, int, int, int);                             \
-  template void launch_dft_xy<T>(bool, int, int, const FastArgs<T>&, hipStream_t);            \
-  template void launch_dft_xy_batch<T>(bool, bool, int, int, int, int, const FastArgs<T>*,    \
-                                       int, int, hipStream_t);                                \
+  template bool dft_values_supported<T>(bool, int, int, int, int, int);                       \
+  template void launch_dft_xy<T>(bool, int, int, int, const FastArgs<T>&, hipStream_t);       \
+  template void launch_dft_xy_batch<T>(bool, bool, int, int, int, int, int,                   \
+                                       const FastArgs<T>*, int, int, hipStream_t);            \
   template void launch_dft_z<T>(bool, int, int, const FastArgs<T>&, hipStream_t);             \
   template void launch_dft_z_batch<T>(bool, bool, int, int, int, int, const FastArgs<T>*,     \
                                       const int2*, int, bool, hipStream_t);

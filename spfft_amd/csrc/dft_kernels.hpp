@@ -99,11 +99,19 @@ void build_dft_tables(void* tables, int nx, int ny, int nz, hipStream_t stream);
 template <typename T>
 bool dft_plane_supported(bool r2c, int nx, int ny, int kx, int ky);
 
+// True when the backward plane kernel can also sum the sticks' values over z
+// itself (sets of stick runs), so that no z kernel is needed.
 template <typename T>
-void launch_dft_xy(bool forward, int nx, int ny, const FastArgs<T>& a, hipStream_t stream);
+bool dft_values_supported(bool r2c, int nx, int ny, int nz, int kx, int ky);
+
+// fromValues: nz for a backward launch from the values (FastArgs::in, hasRuns),
+// 0 from the [z][stick] buffer.
+template <typename T>
+void launch_dft_xy(bool forward, int nx, int ny, int fromValues, const FastArgs<T>& a,
+                   hipStream_t stream);
 // kx, ky (kz below): the batch's largest.
 template <typename T>
-void launch_dft_xy_batch(bool forward, bool r2c, int nx, int ny, int kx, int ky,
+void launch_dft_xy_batch(bool forward, bool r2c, int nx, int ny, int fromValues, int kx, int ky,
                          const FastArgs<T>* batch, int ntrans, int nz, hipStream_t stream);
 
 template <typename T>

@@ -110,6 +110,13 @@ void launch_z(bool forward, int nx, int ny, int nz, const FastArgs<T>& a, hipStr
   }
 }
 
+// Largest set whose backward matrix kernel sums the values over z itself instead
+// of reading a z kernel's output: one launch less, for num_values products per
+// plane and part. FP64 backward, with a z kernel / from the values, us: 20^3 (925
+// values) 9.8 / 6.6, 28^3 (2,517) 10.9 / 8.5, 32^3 (3,743) 9.5 / 9.4, 36^3 (5,257)
+// 9.6 / 10.2; batches of 8: 28^3 11.6 / 9.8, 36^3 13.2 / 18.7.
+constexpr int kFromValues = 3000;
+
 // The plane family to run for `want` among those that serve the shape: the
 // class-split kernels, else the split stage, else the matrix kernels.
 int served_plane(int want, bool classSplit, bool split, bool matrix) {
@@ -219,30 +226,35 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
   tb.classSplit = tb.fast && tb.split &&
                   class_split_supported<T>(map->dimX, map->dimY, tb.numCols, r2c);
   const bool useFast = tb.fast;
-  tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
-  tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
+  // each set's tables are those that its kernels read
   tb.stickBegin = DeviceBuffer<int>::from_host(t.stickBegin);
-  tb.stickY = DeviceBuffer<int>::from_host(t.stickY);
-  tb.stickCol = DeviceBuffer<int>::from_host(t.stickCol);
-  tb.colX = DeviceBuffer<int>::from_host(t.colX);
-  tb.colBegin = DeviceBuffer<int>::from_host(t.colBegin);
+  if (!useFast) {
+    tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
+    tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
+    tb.stickY = DeviceBuffer<int>::from_host(t.stickY);
+    tb.stickCol = DeviceBuffer<int>::from_host(t.stickCol);
+    tb.colBegin = DeviceBuffer<int>::from_host(t.colBegin);
+  }
+  if (!useFast || tb.split) tb.colX = DeviceBuffer<int>::from_host(t.colX);
 
   if (useFast) {
-    // Stick index at (column, y); absent positions, and the extra row
-    // `tb.numCols` used by the lanes past the last column, point at the zero
-    // element that every row of the [z][stick] buffer holds at index nst.
-    // Stored class-interleaved: for column u and j < M = Ny / R the R entries
-    // of y = j + M l (l < R) are adjacent, so a lane of the backward plane
-    // kernel reads all the indices of one decimation-in-frequency output with
-    // R / 4 16-byte loads.
     const int ny = map->dimY;
-    const int R = fast_classes(ny), M = ny / R;
-    std::vector<int> at(static_cast<size_t>(tb.numCols + 1) * ny, map->num_sticks());
-    for (int s = 0; s < map->num_sticks(); ++s) {
-      const int y = t.stickY[s];
-      at[(static_cast<size_t>(t.stickCol[s]) * M + y % M) * R + y / M] = s;
+    if (tb.split) {
+      // Stick index at (column, y); absent positions, and the extra row
+      // `tb.numCols` used by the lanes past the last column, point at the zero
+      // element that every row of the [z][stick] buffer holds at index nst.
+      // Stored class-interleaved: for column u and j < M = Ny / R the R entries
+      // of y = j + M l (l < R) are adjacent, so a lane of the backward plane
+      // kernel reads all the indices of one decimation-in-frequency output with
+      // R / 4 16-byte loads.
+      const int R = fast_classes(ny), M = ny / R;
+      std::vector<int> at(static_cast<size_t>(tb.numCols + 1) * ny, map->num_sticks());
+      for (int s = 0; s < map->num_sticks(); ++s) {
+        const int y = t.stickY[s];
+        at[(static_cast<size_t>(t.stickCol[s]) * M + y % M) * R + y / M] = s;
+      }
+      tb.stickAt = DeviceBuffer<int>::from_host(at);
     }
-    tb.stickAt = DeviceBuffer<int>::from_host(at);
     // tables of the matrix kernels
     if (tb.matrix) {
       const int nx = map->dimX;
@@ -255,6 +267,8 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
         cell[s] = i << 16 | dft::fold_at(ny, tb.ky, y);
         columns[static_cast<size_t>(i) * ny + y] = s;
       }
+      tb.fromValues = map->num_values() <= kFromValues &&
+                      dft_values_supported<T>(r2c, nx, ny, map->dimZ, tb.kx, tb.ky);
       tb.stickCell = DeviceBuffer<int>::from_host(cell);
       tb.columnSticks = DeviceBuffer<int>::from_host(columns);
     }
@@ -311,31 +325,36 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
         runs[st] = make_int4(v0, z0, len, 0);
       }
       if (all) tb.zInfo = DeviceBuffer<int4>::from_host(runs);
+      tb.fromValues = tb.fromValues && all;
     }
-    const int classes = fast_classes(map->dimX);
-    std::vector<int> resBegin(classes + 1, 0), resSticks;
-    resSticks.reserve(map->num_sticks());
-    for (int c = 0; c < classes; ++c) {
-      resBegin[c] = static_cast<int>(resSticks.size());
-      for (int s = 0; s < map->num_sticks(); ++s) {
-        if (t.colX[t.stickCol[s]] % classes == c) resSticks.push_back(s);
+    if (tb.classSplit) {
+      const int classes = fast_classes(map->dimX);
+      std::vector<int> resBegin(classes + 1, 0), resSticks;
+      resSticks.reserve(map->num_sticks());
+      for (int c = 0; c < classes; ++c) {
+        resBegin[c] = static_cast<int>(resSticks.size());
+        for (int s = 0; s < map->num_sticks(); ++s) {
+          if (t.colX[t.stickCol[s]] % classes == c) resSticks.push_back(s);
+        }
       }
+      resBegin[classes] = static_cast<int>(resSticks.size());
+      std::vector<int> resYM(resSticks.size());
+      for (size_t i = 0; i < resSticks.size(); ++i) {
+        const int st = resSticks[i];
+        resYM[i] = (t.stickY[st] << 16) | (t.colX[t.stickCol[st]] / classes);
+      }
+      tb.resYM = DeviceBuffer<int>::from_host(resYM);
+      tb.resSticks = DeviceBuffer<int>::from_host(resSticks);
+      tb.resBegin = DeviceBuffer<int>::from_host(resBegin);
     }
-    resBegin[classes] = static_cast<int>(resSticks.size());
-    std::vector<int> resYM(resSticks.size());
-    for (size_t i = 0; i < resSticks.size(); ++i) {
-      const int st = resSticks[i];
-      resYM[i] = (t.stickY[st] << 16) | (t.colX[t.stickCol[st]] / classes);
+    if (tb.split) {
+      // column of x, or the all-zero column tb.numCols of the xy tile
+      std::vector<int> xCol(map->dimX, tb.numCols);
+      for (int u = 0; u < tb.numCols; ++u) xCol[t.colX[u]] = u;
+      tb.xCol = DeviceBuffer<int>::from_host(xCol);
     }
-    tb.resYM = DeviceBuffer<int>::from_host(resYM);
-    // column of x, or the all-zero column tb.numCols of the xy tile
-    std::vector<int> xCol(map->dimX, tb.numCols);
-    for (int u = 0; u < tb.numCols; ++u) xCol[t.colX[u]] = u;
-    tb.xCol = DeviceBuffer<int>::from_host(xCol);
-    tb.resSticks = DeviceBuffer<int>::from_host(resSticks);
-    tb.resBegin = DeviceBuffer<int>::from_host(resBegin);
     // tile pitch for the whole-plane batch kernels (0: not applicable)
-    if (map->dimX == map->dimY &&
+    if (tb.split && map->dimX == map->dimY &&
         plane_path_supported<T>(map->dimX, tb.numCols, map->type == SPFFT_TRANS_R2C)) {
       tb.pitchT = plane_pitch<T>(map->dimX, tb.numCols);
     }
@@ -571,22 +590,31 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     }
   };
   auto xy_two = [&] { launch_split_xy<T>(forward, map_->dimX, map_->dimY, a, nullptr); };
-  auto xy_matrix = [&] { launch_dft_xy<T>(forward, map_->dimX, map_->dimY, a, nullptr); };
+  // backward from the values the matrix kernels need no z kernel: the other
+  // families are timed with theirs
+  const int fromValues = from_values(forward);
+  auto xy_matrix = [&] {
+    a.hasRuns = f.hasRuns;
+    launch_dft_xy<T>(forward, map_->dimX, map_->dimY, fromValues, a, nullptr);
+  };
   float zr = 0.f, ze = 0.f, fused = 0.f, two = 0.f, matrix = 0.f;
   auto time_z = [&] {
     if (f.hasRuns && fixedZ) {
       zr = time_launches([&] { z(1); }, ev.e0, ev.e1);
       ze = time_launches([&] { z(0); }, ev.e0, ev.e1);
       c.zRuns = zr <= ze ? 1 : 0;
+    } else if (fromValues > 0) {
+      zr = ze = time_launches([&] { z(f.hasRuns); }, ev.e0, ev.e1);
     } else {
       z(f.hasRuns);
     }
   };
   auto time_xy = [&] {
+    const float zTime = fromValues > 0 ? std::min(zr, ze) : 0.f;
     float best = 0.f;
     auto candidate = [&](bool serves, int plane, float* ms, auto&& run) {
       if (!serves) return;
-      *ms = time_launches(run, ev.e0, ev.e1);
+      *ms = time_launches(run, ev.e0, ev.e1) + (plane == 3 ? 0.f : zTime);
       if (best == 0.f || *ms < best) {
         best = *ms;
         c.plane = plane;
@@ -750,15 +778,18 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent) {
     f.out = outGPU;
     const TuneChoice choice =
         single_choice(false, f, stream, inKind != MemKind::Device || hostOut);
-    f.hasRuns = choice.zRuns;
-    launch_z<T>(false, map_->dimX, map_->dimY, map_->dimZ, f, stream);
+    const int fromValues = choice.plane == 3 ? from_values(false) : 0;
+    if (fromValues == 0) {
+      f.hasRuns = choice.zRuns;
+      launch_z<T>(false, map_->dimX, map_->dimY, map_->dimZ, f, stream);
+    }
     // host output: the plane stage runs in chunks of planes, each copied out
     // while the next is computed
     for (int c = 0; c < chunks; ++c) {
       f.zBegin = c * ppc;
       f.nz = std::min(map_->dimZ, (c + 1) * ppc);
       if (choice.plane == 3) {
-        launch_dft_xy<T>(false, map_->dimX, map_->dimY, f, stream);
+        launch_dft_xy<T>(false, map_->dimX, map_->dimY, fromValues, f, stream);
       } else if (choice.plane == 2) {
         launch_split_xy<T>(false, map_->dimX, map_->dimY, f, stream);
       } else {
@@ -845,7 +876,7 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
       f.zBegin = c * ppc;
       f.nz = std::min(map_->dimZ, (c + 1) * ppc);
       if (choice.plane == 3) {
-        launch_dft_xy<T>(true, map_->dimX, map_->dimY, f, stream);
+        launch_dft_xy<T>(true, map_->dimX, map_->dimY, 0, f, stream);
       } else if (choice.plane == 2) {
         launch_split_xy<T>(true, map_->dimX, map_->dimY, f, stream);
       } else {
@@ -931,6 +962,7 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
   shape->maxNcol = 0;
   shape->runs = true;
   shape->classSplit = shape->split = shape->matrix = shape->fixedLengths = true;
+  shape->fromValues = true;
   shape->maxNst = shape->kx = shape->ky = shape->kz = 0;
   for (size_t t = 0; t < n; ++t) {
     const TransformTables<T>& tab = *ex[t]->tab_;
@@ -938,6 +970,7 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
     shape->split = shape->split && ex[t]->split_;
     shape->matrix = shape->matrix && ex[t]->matrix_;
     shape->fixedLengths = shape->fixedLengths && tab.fixedLengths;
+    shape->fromValues = shape->fromValues && tab.fromValues;
     shape->maxNst = std::max(shape->maxNst, ex[t]->map_->num_sticks());
     shape->kx = std::max(shape->kx, tab.kx);
     shape->ky = std::max(shape->ky, tab.ky);
@@ -954,6 +987,9 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
   // the widest columns of different transforms together must fit as well
   shape->matrix = shape->matrix &&
                   dft_plane_supported<T>(shape->r2c, m0.dimX, m0.dimY, shape->kx, shape->ky);
+  shape->fromValues = shape->fromValues && shape->matrix &&
+                      dft_values_supported<T>(shape->r2c, m0.dimX, m0.dimY, m0.dimZ, shape->kx,
+                                              shape->ky);
   return shape->split || shape->matrix;
 }
 
@@ -1013,10 +1049,11 @@ template <typename T>
 void ExecutionGPU<T>::launch_batch(bool forward, const BatchShape& shape, int n,
                                    const TuneChoice& choice, const FastArgs<T>* dArgs,
                                    const int2* dMap, hipStream_t stream) {
+  const int fromValues = !forward && choice.plane == 3 && shape.fromValues ? shape.dimZ : 0;
   auto launch_xy = [&] {
     if (choice.plane == 3) {
-      launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, shape.kx, shape.ky,
-                             dArgs, n, shape.dimZ, stream);
+      launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, fromValues, shape.kx,
+                             shape.ky, dArgs, n, shape.dimZ, stream);
     } else if (choice.plane == 2) {
       launch_split_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, dArgs, n, shape.dimZ,
                                shape.maxNcol, stream);
@@ -1029,7 +1066,7 @@ void ExecutionGPU<T>::launch_batch(bool forward, const BatchShape& shape, int n,
     }
   };
   if (forward) launch_xy();
-  launch_batch_z(forward, shape, choice.zRuns != 0, dArgs, dMap, stream);
+  if (fromValues == 0) launch_batch_z(forward, shape, choice.zRuns != 0, dArgs, dMap, stream);
   if (!forward) launch_xy();
 }
 
@@ -1053,9 +1090,12 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
     launch_split_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, dArgs, n, shape.dimZ,
                              shape.maxNcol, nullptr);
   };
+  // backward from the values the matrix kernels need no z kernel: the other
+  // families are timed with theirs
+  const int fromValues = !forward && shape.fromValues ? shape.dimZ : 0;
   auto xy_matrix = [&] {
-    launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, shape.kx, shape.ky, dArgs,
-                           n, shape.dimZ, nullptr);
+    launch_dft_xy_batch<T>(forward, shape.r2c, shape.dimX, shape.dimY, fromValues, shape.kx,
+                           shape.ky, dArgs, n, shape.dimZ, nullptr);
   };
   // The forward z kernel reads the [z][stick] buffer that the xy kernel
   // writes, the backward xy kernel the one that the z kernel writes.
@@ -1079,7 +1119,10 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
   float split = 0.f, plane0 = 0.f, plane1 = 0.f, two = 0.f, matrix = 0.f;
   float best = 1e30f;
   if (shape.matrix) {
-    best = matrix = time_launches(xy_matrix, ev.e0, ev.e1);
+    // (less the z kernel that it saves)
+    matrix = time_launches(xy_matrix, ev.e0, ev.e1);
+    if (fromValues > 0) matrix -= std::min(zr, ze);
+    best = matrix;
     c.plane = 3;
   }
   if (shape.split) {

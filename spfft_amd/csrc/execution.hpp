@@ -34,6 +34,7 @@ struct TransformTables {
   bool matrix = false;    // the matrix plane kernels do
   bool classSplit = false;    // the class-split plane kernels do (nx = ny, LDS fits)
   bool fixedLengths = false;  // all three lengths are fixed ones
+  bool fromValues = false;    // backward matrix kernels without a z kernel
   int kx = 0, ky = 0, kz = 0;  // largest centred index per dimension
   int numCols = 0;
   int pitchT = 0;  // whole-plane batch kernels' tile pitch (0: not applicable)
@@ -89,6 +90,7 @@ public:
     bool classSplit = false;  // class-split plane kernels serve every transform
     bool split = false, matrix = false;  // the split stage, the matrix kernels do
     bool fixedLengths = false;           // all lengths are fixed ones
+    bool fromValues = false;             // backward matrix kernels without a z kernel
     int maxNst = 0;                      // most sticks
     int kx = 0, ky = 0, kz = 0;          // largest centred indices
     int device = 0;
@@ -165,6 +167,10 @@ private:
                 const hipEvent_t* ready, int readyCount, hipStream_t compute, hipStream_t copy);
   StageArgs<T> base_args() const;
   FastArgs<T> fast_args() const;
+  // nz when the backward matrix kernels take the values themselves, else 0
+  int from_values(bool forward) const {
+    return !forward && tab_->fromValues ? map_->dimZ : 0;
+  }
   // Kernel choices of a single transform (plane stage: class-split, split or
   // matrix kernels; z addressing when the sticks are runs), tuned on the first call
   // of the shape with device input and output, on that call's buffers

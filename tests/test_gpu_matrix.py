@@ -119,3 +119,25 @@ def test_batches(dims, r2c, precision, monkeypatch):
         assert orc.rel_l2(got, o.backward(vals[k])) <= TOL[precision], k
         f = outs[k].cpu().numpy().astype(np.float64).view(np.complex128)
         assert orc.rel_l2(f, o.forward(got, True)) <= TOL[precision], k
+
+
+@pytest.mark.parametrize("precision", ["double", "float"])
+@pytest.mark.parametrize("r2c", [False, True], ids=["c2c", "r2c"])
+@pytest.mark.parametrize("dims", [(20, 20, 20), (21, 19, 23), (24, 24, 24), (16, 16, 2),
+                                  (12, 12, 1), (8, 9, 64)], ids=lambda d: "x".join(map(str, d)))
+def test_backward_from_values(dims, r2c, precision, monkeypatch):
+    """Small sets of stick runs: the plane kernel sums the values over z itself,
+    so no z kernel runs. Also runs that wrap, and whole sticks (z = n / 2 and a
+    hermitian (0,0) stick with both halves given)."""
+    monkeypatch.setenv("SPFFT_AMD_PLANE", "3")
+    seed = 0x5EED1400 + sum(dims)
+    whole = np.stack(np.meshgrid(*[np.arange(n // 2 + 1 if r2c and d == 0 else n)
+                                   for d, n in enumerate(dims)], indexing="ij"), -1)
+    whole = whole.reshape(-1, 3)
+    whole = whole[(whole[:, 0] < 4) & (whole[:, 1] < 5)]
+    for t in (ellipsoid(dims, 0.35, r2c), np.ascontiguousarray(whole.astype(np.int32))):
+        assert len(t) <= 3000
+        tr = check(dims, t, r2c, precision, seed)
+        v = complex_values(seed, len(t))
+        ran = kernels_run(lambda: gpu_backward(tr, v, dims, r2c, precision))
+        assert ran == {"k_xy_backward_dft"}, ran
