@@ -63,5 +63,31 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Before and after the streaming stores of one of two branches: the compiler
+// would hoist or sink the stores of both into one plain store.
+__device__ __forceinline__ void apart() { asm volatile(""); }
+
+// Streaming store (no cache allocation on the way to HBM): for results that no
+// later kernel of the chain reads while they could still be cached.
+template <typename T>
+__device__ __forceinline__ void store_stream(T* p, T v) {
+  __builtin_nontemporal_store(v, p);
+}
+template <typename T>
+__device__ __forceinline__ void store_stream(Cx<T>* p, Cx<T> v) {
+  __builtin_nontemporal_store(v.re, &p->re);
+  __builtin_nontemporal_store(v.im, &p->im);
+}
+
+template <typename T>
+__device__ __forceinline__ T load_stream(const T* p) {
+  return __builtin_nontemporal_load(p);
+}
+template <typename T>
+__device__ __forceinline__ Cx<T> load_stream(const Cx<T>* p) {
+  return Cx<T>{__builtin_nontemporal_load(&p->re), __builtin_nontemporal_load(&p->im)};
+}
+
 }  // namespace dev
+
 }  // namespace spfft

@@ -840,10 +840,18 @@ __device__ __forceinline__ void xy_backward_dft(const FastArgs<T>& a, const Plan
 #pragma unroll
         for (int t = 0; t < TX; ++t) {
           if (t == 0 || xo[t] >= 0) {
+            O value;
             if constexpr (RC) {
-              plane[at + xo[t]] = static_cast<T>(o[t].re);
+              value = static_cast<T>(o[t].re);
             } else {
-              plane[at + xo[t]] = narrow<T>(o[t].re, o[t].im);
+              value = narrow<T>(o[t].re, o[t].im);
+            }
+            if (sizeof(T) == 8 && !RC && a.pastCache) {
+              apart();
+              store_stream(plane + at + xo[t], value);
+              apart();
+            } else {
+              plane[at + xo[t]] = value;
             }
           }
         }

@@ -378,13 +378,6 @@ __host__ __device__ constexpr int tw_offset(int n) {
   return round_up(n, static_cast<int>(sizeof(Tw<T>) / sizeof(Cx<T>)));
 }
 
-// Streaming store (no cache allocation on the way to HBM): for batch outputs
-// that no later kernel of the chain reads while they could still be cached.
-template <typename T>
-__device__ __forceinline__ void store_stream(Cx<T>* p, Cx<T> v) {
-  __builtin_nontemporal_store(v.re, &p->re);
-  __builtin_nontemporal_store(v.im, &p->im);
-}
 // Two consecutive FP32 elements (16 bytes, 16-byte aligned) in one streaming
 // store.
 __device__ __forceinline__ void store_stream_pair(Cx<float>* p, Cx<float> a, Cx<float> b) {
@@ -392,12 +385,33 @@ __device__ __forceinline__ void store_stream_pair(Cx<float>* p, Cx<float> a, Cx<
   const F4 w = {a.re, a.im, b.re, b.im};
   __builtin_nontemporal_store(w, reinterpret_cast<F4*>(p));
 }
-template <bool STREAM, typename T>
-__device__ __forceinline__ void store(Cx<T>* p, Cx<T> v) {
-  if constexpr (STREAM) {
-    store_stream(p, v);
+
+// One lane's E elements of a row of the space domain, P apart, with streaming
+// stores for a large one (see kStreamField).
+template <int E, int P, typename V, typename F>
+__device__ __forceinline__ void store_line(bool stream, V* p, F value) {
+  if (stream) {
+    apart();
+#pragma unroll
+    for (int e = 0; e < E; ++e) store_stream(p + P * e, value(e));
+    apart();
   } else {
-    *p = v;
+#pragma unroll
+    for (int e = 0; e < E; ++e) p[P * e] = value(e);
+  }
+}
+
+// The same for the loads of a row (see kLastLevelCache).
+template <int E, int P, typename V, typename F>
+__device__ __forceinline__ void load_line(bool stream, const V* p, F take) {
+  if (stream) {
+    apart();
+#pragma unroll
+    for (int e = 0; e < E; ++e) take(e, load_stream(p + P * e));
+    apart();
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e) take(e, p[P * e]);
   }
 }
 
@@ -621,7 +635,7 @@ __device__ __forceinline__ void fill_zero_zero_stick(Cx<T>* tile) {
 // first storage z, length}: value of storage z = first + ((z - z0) mod NZ)
 // for the len positions of the run): every lane loads its z values straight
 // into registers, with no entry table, zero fill or scatter.
-template <typename T, int NZ, bool RC, bool STREAM>
+template <typename T, int NZ, bool RC>
 __device__ __forceinline__ void z_backward_runs(const FastArgs<T>& a, int bid) {
   using Z = ZShape<T, NZ>;
   using L = typename Z::L;
@@ -671,13 +685,15 @@ __device__ __forceinline__ void z_backward_runs(const FastArgs<T>& a, int bid) {
   __syncthreads();
   for (int t = threadIdx.x; t < S * NZ; t += NT) {
     const int s = t % S, zz = t / S;
-    if (s < ns) store<STREAM>(&a.zbuf[static_cast<size_t>(zz) * a.pitch + s0 + s], tile[s * LZ + phys<T>(zz)]);
+    if (s < ns) a.zbuf[static_cast<size_t>(zz) * a.pitch + s0 + s] = tile[s * LZ + phys<T>(zz)];
   }
 }
 
-// STREAM: streaming stores of the [z][stick] rows (batches, whose
-// intermediates exceed the caches anyway)
-template <typename T, int NZ, bool RC, bool STREAM>
+// The [z][stick] rows are stored plainly, also for batches: the plane kernel
+// reads them next, and the 256 MiB of last-level cache hold them. (Streaming stores
+// here: 16 transforms of 96^3 FP32 127.8 against 124.6 us per pair of batches,
+// 8 of 128^3 FP64 267 against 262.)
+template <typename T, int NZ, bool RC>
 __device__ __forceinline__ void z_backward_body(const FastArgs<T>& a, int bid) {
   using Z = ZShape<T, NZ>;
   using L = typename Z::L;
@@ -687,7 +703,7 @@ __device__ __forceinline__ void z_backward_body(const FastArgs<T>& a, int bid) {
   const int s0 = bid * S;
   const int ns = min(S, a.nst - s0);
   if (a.hasRuns) {
-    z_backward_runs<T, NZ, RC, STREAM>(a, bid);
+    z_backward_runs<T, NZ, RC>(a, bid);
     return;
   }
   const int e0 = a.stickBegin[s0], e1 = a.stickBegin[s0 + ns];
@@ -755,7 +771,7 @@ __device__ __forceinline__ void z_backward_body(const FastArgs<T>& a, int bid) {
   __syncthreads();
   for (int t = threadIdx.x; t < S * NZ; t += NT) {
     const int s = t % S, zz = t / S;
-    if (s < ns) store<STREAM>(&a.zbuf[static_cast<size_t>(zz) * a.pitch + s0 + s], tile[s * LZ + phys<T>(zz)]);
+    if (s < ns) a.zbuf[static_cast<size_t>(zz) * a.pitch + s0 + s] = tile[s * LZ + phys<T>(zz)];
   }
 }
 
@@ -1086,15 +1102,12 @@ __device__ __forceinline__ void xy_backward_body(const FastArgs<T>& a, int bid) 
       const size_t row = (static_cast<size_t>(z) * N + r + R * ma) * N;
       if (RC) {
         // row b = row a + R rows
-#pragma unroll
-        for (int e = 0; e < LX::E; ++e) {
-          a.out[row + q + LX::P * e] = v[e].re;
-          a.out[row + static_cast<size_t>(R) * N + q + LX::P * e] = v[e].im;
-        }
+        T* rowB = a.out + row + static_cast<size_t>(R) * N;
+        store_line<LX::E, LX::P>(a.streamOut, a.out + row + q, [&](int e) { return v[e].re; });
+        store_line<LX::E, LX::P>(a.streamOut, rowB + q, [&](int e) { return v[e].im; });
       } else {
         Cx<T>* out = reinterpret_cast<Cx<T>*>(a.out) + row;
-#pragma unroll
-        for (int e = 0; e < LX::E; ++e) out[q + LX::P * e] = v[e];
+        store_line<LX::E, LX::P>(a.streamOut, out + q, [&](int e) { return v[e]; });
       }
     }
   }
@@ -1611,16 +1624,11 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   if (y < ny) {
     const size_t row = (static_cast<size_t>(z) * ny + y) * N;
     if (RC) {
-#pragma unroll
-      for (int e = 0; e < E; ++e) a.out[row + q + P * e] = v[e].re;
-      if (hasB) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) a.out[row + N + q + P * e] = v[e].im;
-      }
+      store_line<E, P>(a.streamOut, a.out + row + q, [&](int e) { return v[e].re; });
+      if (hasB) store_line<E, P>(a.streamOut, a.out + row + N + q, [&](int e) { return v[e].im; });
     } else {
       Cx<T>* out = reinterpret_cast<Cx<T>*>(a.out) + row;
-#pragma unroll
-      for (int e = 0; e < E; ++e) out[q + P * e] = v[e];
+      store_line<E, P>(a.streamOut, out + q, [&](int e) { return v[e]; });
     }
   }
 }
@@ -1650,15 +1658,11 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   Cx<T> v[E];
   if (RC) {
     const size_t rowB = hasB ? row + N : row;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const T b = a.in[rowB + q + P * e];
-      v[e] = Cx<T>{a.in[row + q + P * e], hasB ? b : T(0)};
-    }
+    load_line<E, P>(a.pastCache, a.in + row + q, [&](int e, T x) { v[e].re = x; });
+    load_line<E, P>(a.pastCache, a.in + rowB + q, [&](int e, T x) { v[e].im = hasB ? x : T(0); });
   } else {
     const Cx<T>* in = reinterpret_cast<const Cx<T>*>(a.in) + row;
-#pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = in[q + P * e];
+    load_line<E, P>(a.pastCache, in + q, [&](int e, Cx<T> x) { v[e] = x; });
   }
   int uu[E];
 #pragma unroll
@@ -1844,7 +1848,7 @@ __device__ __forceinline__ void full_rows(const FastArgs<T>& a, int z, int line,
 
 template <typename T, int NZ, bool RC>
 __global__ void __launch_bounds__((ZShape<T, NZ>::NT)) k_z_backward_fast(FastArgs<T> a) {
-  z_backward_body<T, NZ, RC, false>(a, blockIdx.x);
+  z_backward_body<T, NZ, RC>(a, blockIdx.x);
 }
 template <typename T, int NZ>
 __global__ void __launch_bounds__((ZShape<T, NZ>::NT)) k_z_forward_fast(FastArgs<T> a) {
@@ -1866,7 +1870,7 @@ __global__ void __launch_bounds__((ZShape<T, NZ>::NT))
   const int2 m = map[blockIdx.x];
   FastArgs<T> a = on_global(batch[m.x], batch);
   a.hasRuns = a.hasRuns && useRuns;
-  z_backward_body<T, NZ, RC, true>(a, m.y);
+  z_backward_body<T, NZ, RC>(a, m.y);
 }
 template <typename T, int NZ>
 __global__ void __launch_bounds__((ZShape<T, NZ>::NT))

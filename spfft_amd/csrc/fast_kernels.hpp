@@ -65,11 +65,13 @@ struct FastArgs {
                                       // every stick's values are one run in user order
   int hasRuns = 0;                    // zInfo is valid (set on the host; kernels select the
                                       // stick-run path on this flag, never on the pointer)
+  int streamOut = 0;                  // backward: streaming stores of the space domain
   const int* xCol = nullptr;          // [NX]: column id of x, or ncol (a zero column)
   const int* resSticks = nullptr;     // sticks grouped by colX mod R
   const int* resBegin = nullptr;      // R + 1 offsets into resSticks
   const int* resYM = nullptr;         // per resSticks entry: y << 16 | (x / R)
   int pitchT = 0;                     // whole-plane kernels: row pitch of the plane tile
+  int pastCache = 0;                  // the launch's space domain is past kLastLevelCache
   Cx<T>* ybuf = nullptr;              // split plane kernels: compact columns [z][y][pitchY]
   int pitchY = 0;                     //   (column u of row y at u; pitchY >= ncol)
   const Tw<T>* twX = nullptr;
@@ -78,6 +80,29 @@ struct FastArgs {
   T scale = T(1);
   int useScale = 0;
 };
+
+// Streaming accesses to the space domain. The last-level cache holds 256 MiB. A
+// launch (one transform, or a batch) that writes less space domain than that leaves
+// it there for the next call to read; more, and the field only pushes out the stick
+// and column buffers that the launch's own kernels pass on, and its write-back falls
+// into the next launch. All times us, plain / streaming stores:
+//   one transform, from 96 MiB: pairs 256^3 FP64 300 / 256, 240^3 FP64 (211 MiB)
+//     289 / 276, 216^3 FP64 (154 MiB) 240 / 238, 256^3 FP32 (128 MiB) 157 / 159;
+//     backward alone 192^3 FP64 (108 MiB) 80 / 72, 256^3 FP32 92 / 70; below that
+//     (128^3 FP64, 32 MiB) 42.4 / 44.5 per pair;
+//   batches, from 144 MiB: 3 x 192^3 FP64 (324 MiB) 399 / 356, 8 x 128^3 FP64
+//     (256 MiB) 240 / 228, 8 x 144^3 FP32 (182 MiB) 280 / 264, 8 x 128^3 R2C
+//     (128 MiB) 154 / 155, 60 x 64^3 R2C (120 MiB) 142 / 148.
+// The matrix kernels write tiles of 16 columns: 256-byte segments for FP64 C2C, which
+// stream once the space domain is past the cache (12 x 120^3, 316 MiB, 365 / 342; 11 x
+// 100^3, 168 MiB, 192 / 218), 128 and 64 bytes for the other types, which stay plain
+// (12 x 120^3 R2C 226 / 251).
+constexpr size_t kStreamField = size_t{96} << 20;
+constexpr size_t kStreamBatch = size_t{144} << 20;
+// Forward: the split stage's x kernel reads a space domain past the cache with
+// streaming loads, which keep it out of the column buffer's way (256^3 FP64 pair 266
+// / 255 us plain / streaming; within the cache, 224^3 FP64, 237 / 240).
+constexpr size_t kLastLevelCache = size_t{256} << 20;
 
 // Residue classes per plane used by the xy kernels of length n.
 // (A divisor of n: the stick index table is class-interleaved with it.)
