@@ -279,9 +279,10 @@ def launch_floor(torch, kernel_us):
 
 def plain_lengths_bench(args, sp, torch, np):
     """Single C2C FP64 transforms at other plane-wave lengths, sphere radius
-    0.3125 N (40 at 128): 120, 100, 144 and 132 (z kernels and the split plane
-    stage; 120, 100 and 132 on mixed radix schedules, 132 with a radix-11
-    pass) and 143 (11 x 13: generic stage kernels). Backward+forward pairs/s
+    0.3125 N (40 at 128): 120, 100, 144 and 132 (fixed-length z kernels, the
+    split plane stage or the matrix kernels, as the tuner chooses; 120, 100
+    and 132 on mixed radix schedules, 132 with a radix-11 pass) and 143 (11 x
+    13: matrix kernels). Backward+forward pairs/s
     and the fraction of the HBM roofline of the pair's compulsory bytes,
     rotating over 8 transforms; `kernels` names the kernels one pair
     launched."""
@@ -319,8 +320,8 @@ def plain_lengths_bench(args, sp, torch, np):
         torch.cuda.synchronize()
         kernels = sorted(read_profile(sp.lib))
         sp.lib.spfft_amd_profiling_enable(0)
-        path = "fixed-length" if any(k.startswith("k_z_backward_") and k != "k_z_backward"
-                                     for k in kernels) else "generic"
+        path = ("generic" if "k_z_backward" in kernels else
+                "matrix" if any(k.endswith("_dft") for k in kernels) else "fixed-length")
         pair_bytes = 2 * (20 * len(t) + 16 * n ** 3)
         out[f"{n}^3"] = {"values": len(t), "pairs_per_s": rate,
                          "frac_hbm_wall": pair_bytes * rate / 1e9 / HBM_PEAK_GBS,

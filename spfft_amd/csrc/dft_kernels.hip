@@ -28,7 +28,8 @@
 // (plane kernels) or per backward + forward pair, against the kernels they
 // replace: plane stage at 100^3 backward 20.7 -> 13.7, forward 20.5 -> 11.1
 // (split stage); six bands of 60^3 26 -> 14, 24 -> 13; pair at 97^3 804 -> 39,
-// 67^3 529 -> 27, 20^3 35 -> 18 (generic kernels). At 100^3 the plane kernels
+// 67^3 529 -> 27, 20^3 35 -> 18 (generic kernels; 14.7 with the sums over z in the
+// plane kernel). At 100^3 the plane kernels
 // write 16 MB in 13.7 us: bound by the two chains load - sum - store; the sums
 // alone take 2.6 us of the matrix cores. From about 128 points on the sums
 // dominate (their work per line grows with its length squared) and the fixed-
