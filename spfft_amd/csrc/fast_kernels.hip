@@ -544,6 +544,53 @@ __device__ __forceinline__ void wave_fft(Cx<T>* v, Cx<T>* line, int es, int q,
   }
 }
 
+// The FFT of a line (dividing schedules) whose exchanges go through LDS in two
+// halves, the real parts, then the imaginary parts: `line` holds N reals (padded
+// as 8-byte elements) instead of N complex elements.
+template <typename T, int N, bool BWD, int E, int NS = 1>
+__device__ __forceinline__ void wave_fft_half(Cx<T>* v, T* line, int q,
+                                              const Tw<T>* __restrict__ tw) {
+  constexpr int PL = N / E;
+  constexpr int R = wave_radix(N / NS, E);
+  constexpr int EB = E / R;
+  constexpr int STEP = N / (NS * R);
+#pragma unroll
+  for (int b = 0; b < EB; ++b) {
+    Cx<T> u[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) u[r] = v[b + r * EB];
+    if constexpr (NS > 1) {
+      const int k = (q + PL * b) % NS;
+#pragma unroll
+      for (int r = 1; r < R; ++r) u[r] = cmul(u[r], twiddle<BWD>(tw, k * r * STEP));
+    }
+    Butterfly<T, R, BWD>::run(u, tw, N);
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[b + r * EB] = u[r];
+  }
+  if constexpr (NS * R != N) {
+    auto put = [&](auto part) {
+#pragma unroll
+      for (int b = 0; b < EB; ++b) {
+        const int j = q + PL * b, o = (j / NS) * NS * R + (j % NS);
+#pragma unroll
+        for (int r = 0; r < R; ++r) line[phys<float>(o + r * NS)] = part(v[b + r * EB]);
+      }
+      wave_sync();
+    };
+    T re[E];
+    put([](const Cx<T>& x) { return x.re; });
+#pragma unroll
+    for (int e = 0; e < E; ++e) re[e] = line[phys<float>(q + PL * e)];
+    wave_sync();
+    put([](const Cx<T>& x) { return x.im; });
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = Cx<T>{re[e], line[phys<float>(q + PL * e)]};
+    wave_sync();
+    wave_fft_half<T, N, BWD, E, NS * R>(v, line, q, tw);
+  }
+}
+
 // One output of the decimation-in-frequency split over R inputs x[l] with
 // the class's twiddles w[l] = W_R^(+-r l): sum_l w[l] x[l]. For R = 4 the
 // twiddles are 1, w1, w2 = +-1, w3 = conj(w1), and the sum needs 10 real
@@ -1470,7 +1517,26 @@ struct SplitShape {
   // lanes (P not dividing the wave)
   static constexpr int XL = LINES + (L::SPARE ? NW : 0);
   // the exchange regions, reused as the tile between phases
-  static constexpr int REGION = XL * LB > N * TP ? XL * LB : N * TP;
+  static constexpr int FULL = XL * LB > N * TP ? XL * LB : N * TP;
+  // Halved regions (wave_fft_half, and the tile in two halves of its rows): for
+  // FP64 lines whose full regions leave a CU at most 12 waves, since a launch is
+  // rounds of resident workgroups of about equal time. 192^3 C2C (radius 0.25 N),
+  // 8 waves, 16 with the halves: y kernels 25.8 -> 21.4 and 24.9 -> 21.3 us, x
+  // kernels 29.3 -> 28.1 and 29.3 -> 30.3, pair 133 -> 127; 192^3 R2C pair 94 ->
+  // 84, 200^3 C2C 183 -> 165, 216^3 238 -> 212; 256^3 (12 waves; radius 0.31 N) 288
+  // -> 285. Launches of one round do not gain: 96^3 48.3 -> 51.2, 128^3 even. Nor do
+  // the x kernels of longer lines, which run at the copy rate (320^3 backward 159 us
+  // full, 178 halved; 384^3 279, 302).
+  static constexpr int WAVES = static_cast<int>(
+      kLdsMax / (static_cast<size_t>(tw_offset<T>(FULL)) * sizeof(Cx<T>) + N * sizeof(Tw<T>) +
+                 N * sizeof(Cx<T>)) * NW);
+  static constexpr bool HALF_Y =
+      sizeof(T) == 8 && N > 128 && dividing_schedule(N, L::E) && L::E % 2 == 0 && WAVES <= 12;
+  static constexpr bool HALF_X = HALF_Y && N <= 256;
+  static constexpr int LBH = padded_len<float>(N);   // a line's halved region, in reals
+  static constexpr int XH = (XL * LBH + 1) / 2;
+  static constexpr int REGION_Y = !HALF_Y ? FULL : (XH > N / 2 * TP ? XH : N / 2 * TP);
+  static constexpr int REGION_X = HALF_X ? XH : FULL;
   // This lane's line in the workgroup (LINES for a spare lane: none) and the
   // exchange region it runs in.
   __device__ static int line_of(int wave, int lane) {
@@ -1478,7 +1544,21 @@ struct SplitShape {
   }
   template <typename C>
   __device__ static C* xregion(C* region, int wave, int lane) {
-    return region + (L::spare(lane) ? LINES + wave : wave * L::PER_WAVE + lane / L::P) * LB;
+    return region + region_of(wave, lane) * LB;
+  }
+  __device__ static int region_of(int wave, int lane) {
+    return L::spare(lane) ? LINES + wave : wave * L::PER_WAVE + lane / L::P;
+  }
+  __device__ static T* hregion(Cx<T>* region, int wave, int lane) {
+    return reinterpret_cast<T*>(region) + region_of(wave, lane) * LBH;
+  }
+  template <bool BWD, bool HALF>
+  __device__ static void fft(Cx<T>* v, Cx<T>* region, int wave, int lane, const Tw<T>* tw) {
+    if constexpr (HALF) {
+      wave_fft_half<T, N, BWD, L::E>(v, hregion(region, wave, lane), lane % L::P, tw);
+    } else {
+      wave_fft<T, N, BWD, 1, L::E>(v, xregion(region, wave, lane), 1, lane % L::P, tw);
+    }
   }
   // rows per workgroup of the row kernels (rows of length N): R2C packs two
   // real rows into each complex line
@@ -1487,10 +1567,12 @@ struct SplitShape {
   __host__ __device__ static int row_groups(int ny, bool rc) {
     return (ny + row_block(rc) - 1) / row_block(rc);
   }
-  // region, twiddles, the filled x = 0 column (R2C backward)
-  static constexpr size_t lds() {
-    return static_cast<size_t>(tw_offset<T>(REGION)) * sizeof(Cx<T>) + N * sizeof(Tw<T>) +
-           N * sizeof(Cx<T>);
+  // region, twiddles, the filled x = 0 column (R2C backward). The full regions
+  // of the x kernels need less, but two workgroups per CU instead of three suit
+  // the rows they store (512^3 backward 573 / 642 us).
+  static constexpr size_t lds(bool y) {
+    return static_cast<size_t>(tw_offset<T>(y ? REGION_Y : REGION_X)) * sizeof(Cx<T>) +
+           N * sizeof(Tw<T>) + N * sizeof(Cx<T>);
   }
   __host__ __device__ static int col_groups(int ncol) { return (ncol + LINES - 1) / LINES; }
 };
@@ -1513,7 +1595,7 @@ __device__ __forceinline__ void ysplit_backward_body(const FastArgs<T>& a, int b
   const int u0 = (bid % groups) * S::LINES;
   if (z >= a.nz) return;
   Cx<T>* region = reinterpret_cast<Cx<T>*>(spfft_lds_fast);
-  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION));
+  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION_Y));
   Cx<T>* fill = reinterpret_cast<Cx<T>*>(twl + N);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int q = lane % P;
@@ -1552,19 +1634,27 @@ __device__ __forceinline__ void ysplit_backward_body(const FastArgs<T>& a, int b
   } else {
     __syncthreads();  // twiddles
   }
-  Cx<T>* lr = S::xregion(region, wave, lane);
-  wave_fft<T, N, true, 1, E>(v, lr, 1, q, twl);
-  __syncthreads();  // the exchange regions become the tile
-  if (line < S::LINES) {
-#pragma unroll
-    for (int e = 0; e < E; ++e) region[(q + P * e) * S::TP + line] = v[e];
-  }
-  __syncthreads();
+  S::template fft<true, S::HALF_Y>(v, region, wave, lane, twl);
   Cx<T>* yrows = a.ybuf + static_cast<size_t>(z) * N * a.pitchY + u0;
   const int nc = min(S::LINES, a.ncol - u0);
-  for (int t = threadIdx.x; t < N * S::LINES; t += S::NT) {
-    const int y = t / S::LINES, c = t - y * S::LINES;
-    if (c < nc) yrows[static_cast<size_t>(y) * a.pitchY + c] = region[y * S::TP + c];
+  // the tile, in one part or two (rows below and from N / 2: e below and from E / 2)
+  constexpr int H = S::HALF_Y ? 2 : 1;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    __syncthreads();  // the exchange regions (the last part) become the tile
+    if (line < S::LINES) {
+#pragma unroll
+      for (int e = 0; e < E / H; ++e) {
+        region[(q + P * e) * S::TP + line] = v[e + h * (E / H)];
+      }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < N / H * S::LINES; t += S::NT) {
+      const int y = t / S::LINES, c = t - y * S::LINES;
+      if (c < nc) {
+        yrows[static_cast<size_t>(y + h * (N / H)) * a.pitchY + c] = region[y * S::TP + c];
+      }
+    }
   }
 }
 
@@ -1579,7 +1669,7 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   const int y0 = (bid % groups) * S::row_block(RC);
   if (z >= a.nz) return;
   Cx<T>* region = reinterpret_cast<Cx<T>*>(spfft_lds_fast);
-  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION));
+  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION_X));
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int q = lane % P;
   const int line = S::line_of(wave, lane);
@@ -1620,7 +1710,7 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   }
   for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twX[t];
   __syncthreads();
-  wave_fft<T, N, true, 1, E>(v, S::xregion(region, wave, lane), 1, q, twl);
+  S::template fft<true, S::HALF_X>(v, region, wave, lane, twl);
   if (y < ny) {
     const size_t row = (static_cast<size_t>(z) * ny + y) * N;
     if (RC) {
@@ -1644,7 +1734,7 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   const int y0 = (bid % groups) * S::row_block(RC);
   if (z >= a.nz) return;
   Cx<T>* region = reinterpret_cast<Cx<T>*>(spfft_lds_fast);
-  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION));
+  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION_X));
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int q = lane % P;
   const int line = S::line_of(wave, lane);
@@ -1669,24 +1759,51 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   for (int e = 0; e < E; ++e) uu[e] = a.xCol[q + P * e];
   for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twX[t];
   __syncthreads();
-  Cx<T>* lr = S::xregion(region, wave, lane);
-  wave_fft<T, N, false, 1, E>(v, lr, 1, q, twl);
+  S::template fft<false, S::HALF_X>(v, region, wave, lane, twl);
   if (RC) {
     // Z = A + i B with A, B the spectra of the real rows a and b:
     // A[x] = (Z[x] + conj Z[N - x]) / 2, B[x] = -i (Z[x] - conj Z[N - x]) / 2.
     // The partner of x is held by lane (P - q) % P; it comes through the
-    // line's exchange region (wave-local).
+    // line's exchange region (wave-local; real, then imaginary parts in a
+    // halved one).
+    Cx<T> partner[E];
     wave_sync();
+    if constexpr (S::HALF_X) {
+      T* lr = S::hregion(region, wave, lane);
 #pragma unroll
-    for (int e = 0; e < E; ++e) lr[phys<T>(q + P * e)] = v[e];
-    wave_sync();
+      for (int e = 0; e < E; ++e) lr[phys<float>(q + P * e)] = v[e].re;
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int x = q + P * e;
+        partner[e].re = lr[phys<float>(x == 0 ? 0 : N - x)];
+      }
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < E; ++e) lr[phys<float>(q + P * e)] = v[e].im;
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int x = q + P * e;
+        partner[e].im = lr[phys<float>(x == 0 ? 0 : N - x)];
+      }
+    } else {
+      Cx<T>* lr = S::xregion(region, wave, lane);
+#pragma unroll
+      for (int e = 0; e < E; ++e) lr[phys<T>(q + P * e)] = v[e];
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int x = q + P * e;
+        partner[e] = lr[phys<T>(x == 0 ? 0 : N - x)];
+      }
+    }
     if (y < ny) {
       Cx<T>* ya = a.ybuf + (static_cast<size_t>(z) * ny + y) * a.pitchY;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const int x = q + P * e;
         if (uu[e] < a.ncol) {
-          const Cx<T> zp = lr[phys<T>(x == 0 ? 0 : N - x)];
+          const Cx<T> zp = partner[e];
           const T h = T(0.5);
           ya[uu[e]] = Cx<T>{h * (v[e].re + zp.re), h * (v[e].im - zp.im)};
           if (hasB) ya[a.pitchY + uu[e]] = Cx<T>{h * (v[e].im + zp.im), h * (zp.re - v[e].re)};
@@ -1712,7 +1829,7 @@ __device__ __forceinline__ void ysplit_forward_body(const FastArgs<T>& a, int bi
   const int u0 = (bid % groups) * S::LINES;
   if (z >= a.nz) return;
   Cx<T>* region = reinterpret_cast<Cx<T>*>(spfft_lds_fast);
-  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION));
+  Tw<T>* twl = reinterpret_cast<Tw<T>*>(region + tw_offset<T>(S::REGION_Y));
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int q = lane % P;
   const int line = S::line_of(wave, lane);
@@ -1722,32 +1839,46 @@ __device__ __forceinline__ void ysplit_forward_body(const FastArgs<T>& a, int bi
   // ncol are zero. Thread t holds column t % LINES of rows t / LINES + P k,
   // k < E (N LINES = E NT), all loads in flight before the tile stores.
   const Cx<T>* yrows = a.ybuf + static_cast<size_t>(z) * N * a.pitchY + u0;
-  if constexpr (N * S::LINES != E * S::NT || S::NT % S::LINES != 0) {
-    // spare lanes: no whole-tile thread mapping
-    for (int t = threadIdx.x; t < N * S::LINES; t += S::NT) {
-      const int y = t / S::LINES, c = t - y * S::LINES;
-      region[y * S::TP + c] =
-          c < nc ? yrows[static_cast<size_t>(y) * a.pitchY + c] : Cx<T>{T(0), T(0)};
-    }
-  } else {
-    constexpr int RS = S::NT / S::LINES;  // rows per pass of the workgroup
-    const int c = threadIdx.x % S::LINES, y0 = threadIdx.x / S::LINES;
-    const int cc = c < nc ? c : 0;
-    Cx<T> w[E];
+  // (in one part or two, as in the backward kernel)
+  constexpr int H = S::HALF_Y ? 2 : 1;
+  constexpr bool WHOLE = N * S::LINES == E * S::NT && S::NT % S::LINES == 0;
+  constexpr int RS = S::NT / S::LINES;  // rows per pass of the workgroup
+  const int c0 = threadIdx.x % S::LINES, y0 = threadIdx.x / S::LINES;
+  Cx<T> w[WHOLE ? E : 1];
+  if constexpr (WHOLE) {
+    const int cc = c0 < nc ? c0 : 0;
 #pragma unroll
     for (int k = 0; k < E; ++k) w[k] = yrows[static_cast<size_t>(y0 + RS * k) * a.pitchY + cc];
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-      region[(y0 + RS * k) * S::TP + c] = c < nc ? w[k] : Cx<T>{T(0), T(0)};
-    }
   }
-  for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twY[t];
-  __syncthreads();
   Cx<T> v[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = region[(q + P * e) * S::TP + (line < S::LINES ? line : 0)];
+  for (int h = 0; h < H; ++h) {
+    if (h > 0) __syncthreads();  // the first part has been read
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int k = 0; k < E / H; ++k) {
+        region[(y0 + RS * k) * S::TP + c0] = c0 < nc ? w[k + h * (E / H)] : Cx<T>{T(0), T(0)};
+      }
+    } else {
+      // spare lanes: no whole-tile thread mapping
+      for (int t = threadIdx.x; t < N / H * S::LINES; t += S::NT) {
+        const int y = t / S::LINES, c = t - y * S::LINES;
+        region[y * S::TP + c] =
+            c < nc ? yrows[static_cast<size_t>(y + h * (N / H)) * a.pitchY + c]
+                   : Cx<T>{T(0), T(0)};
+      }
+    }
+    if (h == 0) {
+      for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twY[t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E / H; ++e) {
+      v[e + h * (E / H)] = region[(q + P * e) * S::TP + (line < S::LINES ? line : 0)];
+    }
+  }
   __syncthreads();  // the tile becomes the exchange regions
-  wave_fft<T, N, false, 1, E>(v, S::xregion(region, wave, lane), 1, q, twl);
+  S::template fft<false, S::HALF_Y>(v, region, wave, lane, twl);
   if (u < a.ncol) {
     Cx<T>* zrow = a.zbuf + static_cast<size_t>(z) * a.pitch;
 #pragma unroll
@@ -2561,12 +2692,12 @@ int plane_xy_slots(bool forward, int n) {
 
 // ---- split plane stage launches
 
-template <typename T, int N, typename Kernel, typename... Args>
+template <typename T, int N, bool Y, typename Kernel, typename... Args>
 void split_launch(Kernel kernel, const char* name, int blocks, hipStream_t stream, Args... args) {
   using S = SplitShape<T, N>;
-  prepare_lds(kernel, S::lds());
+  prepare_lds(kernel, S::lds(Y));
   prof::KernelSpan span(stream, name, true);
-  hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(S::NT), S::lds(), stream, span.start(),
+  hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(S::NT), S::lds(Y), stream, span.start(),
                         span.stop(), 0, args...);
   check_launch();
 }
@@ -2578,10 +2709,11 @@ void ysplit_n(bool forward, const FastArgs<T>& a, hipStream_t stream) {
   using S = SplitShape<T, NY>;
   const int blocks = S::col_groups(a.ncol) * (a.nz - a.zBegin);
   if (forward) {
-    split_launch<T, NY>(k_ysplit_forward<T, NY>, "k_ysplit_forward", blocks, stream, a);
+    split_launch<T, NY, true>(k_ysplit_forward<T, NY>, "k_ysplit_forward", blocks, stream, a);
   } else {
-    split_launch<T, NY>(a.r2c ? k_ysplit_backward<T, NY, true> : k_ysplit_backward<T, NY, false>,
-                        "k_ysplit_backward", blocks, stream, a);
+    split_launch<T, NY, true>(
+        a.r2c ? k_ysplit_backward<T, NY, true> : k_ysplit_backward<T, NY, false>,
+        "k_ysplit_backward", blocks, stream, a);
   }
 }
 template <typename T, int NX>
@@ -2589,11 +2721,13 @@ void xsplit_n(bool forward, const FastArgs<T>& a, hipStream_t stream) {
   using S = SplitShape<T, NX>;
   const int blocks = S::row_groups(a.ny, a.r2c != 0) * (a.nz - a.zBegin);
   if (forward) {
-    split_launch<T, NX>(a.r2c ? k_xsplit_forward<T, NX, true> : k_xsplit_forward<T, NX, false>,
-                        "k_xsplit_forward", blocks, stream, a);
+    split_launch<T, NX, false>(
+        a.r2c ? k_xsplit_forward<T, NX, true> : k_xsplit_forward<T, NX, false>,
+        "k_xsplit_forward", blocks, stream, a);
   } else {
-    split_launch<T, NX>(a.r2c ? k_xsplit_backward<T, NX, true> : k_xsplit_backward<T, NX, false>,
-                        "k_xsplit_backward", blocks, stream, a);
+    split_launch<T, NX, false>(
+        a.r2c ? k_xsplit_backward<T, NX, true> : k_xsplit_backward<T, NX, false>,
+        "k_xsplit_backward", blocks, stream, a);
   }
 }
 template <typename T, int NY>
@@ -2602,10 +2736,10 @@ void ysplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans,
   using S = SplitShape<T, NY>;
   const int per = S::col_groups(maxNcol) * nz;
   if (forward) {
-    split_launch<T, NY>(k_ysplit_forward_batch<T, NY>, "k_ysplit_forward_batch", per * ntrans,
+    split_launch<T, NY, true>(k_ysplit_forward_batch<T, NY>, "k_ysplit_forward_batch", per * ntrans,
                         stream, batch, per);
   } else {
-    split_launch<T, NY>(rc ? k_ysplit_backward_batch<T, NY, true>
+    split_launch<T, NY, true>(rc ? k_ysplit_backward_batch<T, NY, true>
                            : k_ysplit_backward_batch<T, NY, false>,
                         "k_ysplit_backward_batch", per * ntrans, stream, batch, per);
   }
@@ -2616,11 +2750,11 @@ void xsplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans,
   using S = SplitShape<T, NX>;
   const int per = S::row_groups(ny, rc) * nz;
   if (forward) {
-    split_launch<T, NX>(rc ? k_xsplit_forward_batch<T, NX, true>
+    split_launch<T, NX, false>(rc ? k_xsplit_forward_batch<T, NX, true>
                            : k_xsplit_forward_batch<T, NX, false>,
                         "k_xsplit_forward_batch", per * ntrans, stream, batch, per);
   } else {
-    split_launch<T, NX>(rc ? k_xsplit_backward_batch<T, NX, true>
+    split_launch<T, NX, false>(rc ? k_xsplit_backward_batch<T, NX, true>
                            : k_xsplit_backward_batch<T, NX, false>,
                         "k_xsplit_backward_batch", per * ntrans, stream, batch, per);
   }
