@@ -6,6 +6,9 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
+# kernel choices of this run only: a file left by another program would decide
+# which kernels the tests reach (tests of the file name their own)
+os.environ.setdefault("SPFFT_AMD_TUNE_CACHE", "off")
 
 
 def pytest_configure(config):
