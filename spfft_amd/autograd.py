@@ -41,6 +41,8 @@ sp.lib.spfft_amd_field_energy.argtypes = [_i, _vp, _vp, _ll, _i, _vp, _vp, _vp]
 sp.lib.spfft_amd_field_energy.restype = _i
 sp.lib.spfft_amd_energy_field.argtypes = [_i, _vp, _vp, _vp, _ll, _i, _vp, _vp]
 sp.lib.spfft_amd_energy_field.restype = _i
+sp.lib.spfft_amd_float_backward_fft.argtypes = [_i] + 3 * [ctypes.POINTER(_vp)]
+sp.lib.spfft_amd_float_backward_fft.restype = _i
 
 
 def _dtype(transform):
@@ -165,7 +167,17 @@ def _rows(x):
     return [x.data_ptr() + b * step for b in range(x.shape[0])]
 
 
-def _batch_backward(transforms, dims, C):
+def _float_backward_fft(transforms, inputs, outputs):
+    array = _vp * len(transforms)
+    sp._check(sp.lib.spfft_amd_float_backward_fft(
+        len(transforms), array(*[t.handle for t in transforms]), array(*inputs),
+        array(*outputs)), "float_backward_fft")
+
+
+def _batch_backward(transforms, dims, C, for_energy=False):
+    """The bands' fields. for_energy: FP32 fields from FFT kernels alone. Their
+    rounding is that of the energy, which is a float64 sum over them: the matrix
+    kernels round differently, and would move it by a few 1e-7 of itself."""
     nx, ny, nz = dims
     n = transforms[0].num_values
     for t in transforms:
@@ -178,7 +190,10 @@ def _batch_backward(transforms, dims, C):
     C = C.contiguous()
     psi = torch.empty((len(transforms), nz, ny, nx), dtype=C.dtype, device=C.device)
     with _OnDefaultStream():
-        sp.multi_transform_backward(transforms, _rows(C), _rows(psi))
+        if for_energy and C.dtype == torch.complex64:
+            _float_backward_fft(transforms, _rows(C), _rows(psi))
+        else:
+            sp.multi_transform_backward(transforms, _rows(C), _rows(psi))
     return psi
 
 
@@ -252,7 +267,7 @@ def _energy_gradient(transforms, psi, own, potential, grad_energy):
 class SparseEnergyBatch(torch.autograd.Function):
     @staticmethod
     def forward(ctx, C, potential, transforms, dims, recompute="auto", memory_budget=None):
-        psi = _batch_backward(transforms, dims, C)
+        psi = _batch_backward(transforms, dims, C, for_energy=True)
         energy = _band_energy(psi, potential)
         ctx.transforms, ctx.dims = transforms, dims
         ctx.recompute = recompute_fields(psi.numel() * psi.element_size(), recompute,
@@ -277,5 +292,6 @@ class SparseEnergyBatch(torch.autograd.Function):
 def sparse_energy_batch(C, potential, transforms, dims, recompute="auto", memory_budget=None):
     """sum_b sum_r V |psi_b|^2 over the bands' transforms (C: bands x values),
     accumulated and returned in float64 for either precision; the gradient has
-    C's dtype."""
+    C's dtype. The energy of complex64 bands carries the FP32 rounding of their
+    fields and densities: it is good to single precision."""
     return SparseEnergyBatch.apply(C, potential, transforms, dims, recompute, memory_budget)

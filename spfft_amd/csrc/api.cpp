@@ -101,18 +101,20 @@ public:
   }
 
   static void backward(int n, TransformType* transforms, const ValueType* const* inputs,
-                       ValueType* const* outputs) {
+                       ValueType* const* outputs, Families families = Families::kAll) {
     check(n, transforms);
     {
       std::vector<TransformInternal<ValueType>*> ts;
       for (int t = 0; t < n; ++t) ts.push_back(transforms[t].transform_.get());
       if (TransformInternal<ValueType>::batch_backward(
               ts, std::vector<const ValueType*>(inputs, inputs + n),
-              std::vector<ValueType*>(outputs, outputs + n))) {
+              std::vector<ValueType*>(outputs, outputs + n), families)) {
         return;
       }
     }
-    for (int t = 0; t < n; ++t) transforms[t].transform_->backward_enqueue(inputs[t], outputs[t]);
+    for (int t = 0; t < n; ++t) {
+      transforms[t].transform_->backward_enqueue(inputs[t], outputs[t], families);
+    }
     for (int t = 0; t < n; ++t) transforms[t].transform_->synchronize();
   }
 
@@ -517,6 +519,19 @@ SpfftError spfft_amd_multi_transform_noalloc(int numTransforms, SpfftTransform* 
   return guarded([&] {
     spfft::MultiTransformInternal<spfft::Transform>::noalloc(
         numTransforms, transforms, inputPointers, outputPointers, forward != 0, scalingTypes);
+  });
+}
+
+// Hook of spfft_amd/autograd.py (no counterpart in the reference ABI):
+// spfft_float_multi_transform_backward_ptr for C2C transforms without the matrix
+// kernels.
+__attribute__((visibility("default"))) SpfftError spfft_amd_float_backward_fft(
+    int numTransforms, SpfftFloatTransform* transforms, const float* const* inputPointers,
+    float* const* outputPointers) {
+  return guarded([&] {
+    auto ts = gather<spfft::TransformFloat>(numTransforms, transforms);
+    spfft::MultiTransformInternal<spfft::TransformFloat>::backward(
+        numTransforms, ts.data(), inputPointers, outputPointers, spfft::Families::kFft);
   });
 }
 

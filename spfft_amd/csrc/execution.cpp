@@ -228,14 +228,16 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
   const bool useFast = tb.fast;
   // each set's tables are those that its kernels read
   tb.stickBegin = DeviceBuffer<int>::from_host(t.stickBegin);
-  if (!useFast) {
+  // The energy of FP32 bands takes its fields from FFT kernels (Families::kFft).
+  tb.generic = !useFast || (sizeof(T) == 4 && !r2c && !tb.fixedLengths);
+  if (tb.generic) {
     tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
     tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
     tb.stickY = DeviceBuffer<int>::from_host(t.stickY);
     tb.stickCol = DeviceBuffer<int>::from_host(t.stickCol);
     tb.colBegin = DeviceBuffer<int>::from_host(t.colBegin);
   }
-  if (!useFast || tb.split) tb.colX = DeviceBuffer<int>::from_host(t.colX);
+  if (tb.generic || tb.split) tb.colX = DeviceBuffer<int>::from_host(t.colX);
 
   if (useFast) {
     const int ny = map->dimY;
@@ -547,14 +549,16 @@ FastArgs<T> ExecutionGPU<T>::fast_args() const {
 
 template <typename T>
 TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream,
-                                          bool staged) {
+                                          bool staged, Families families) {
   TuneChoice c;
   c.zRuns = f.hasRuns;
   const int forced = plane_kernels_forced();
+  const bool fft = families == Families::kFft;
+  const bool mayMatrix = matrix_ && !fft;
   // single transforms have no whole-plane kernels; x != y planes and lengths
   // without class-split kernels only the split stage and the matrix kernels,
   // lengths that are not fixed only the latter
-  c.plane = served_plane(forced, classSplit_, split_, matrix_);
+  c.plane = served_plane(forced, classSplit_, split_, mayMatrix);
   if (forced >= 0) return c;
   // batched fallbacks on the transform's own stream keep the defaults
   if (stream != nullptr) return c;
@@ -563,11 +567,11 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   if (!split_ && !(fixedZ && f.hasRuns)) return c;
   const TuneKey key = make_tune_key(grid_->device_id(), static_cast<int>(sizeof(T)), map_->dimX,
                                     map_->dimY, map_->dimZ, map_->type == SPFFT_TRANS_R2C,
-                                    forward, numCols_, map_->num_sticks(), 1);
+                                    forward, fft, numCols_, map_->num_sticks(), 1);
   TuneChoice known;
   if (tune_lookup(key, &known)) {
     c.zRuns = known.zRuns && f.hasRuns;
-    c.plane = served_plane(known.plane, classSplit_, split_, matrix_);
+    c.plane = served_plane(known.plane, classSplit_, split_, mayMatrix);
     return c;
   }
   // Host data staged in the work buffer, which the split stage's candidate
@@ -595,7 +599,7 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   auto xy_two = [&] { launch_split_xy<T>(forward, map_->dimX, map_->dimY, a, nullptr); };
   // backward from the values the matrix kernels need no z kernel: the other
   // families are timed with theirs
-  const int fromValues = from_values(forward);
+  const int fromValues = mayMatrix ? from_values(forward) : 0;
   auto xy_matrix = [&] {
     a.hasRuns = f.hasRuns;
     launch_dft_xy<T>(forward, map_->dimX, map_->dimY, fromValues, a, nullptr);
@@ -625,7 +629,7 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     };
     candidate(classSplit_, 0, &fused, xy_fused);
     candidate(split_, 2, &two, xy_two);
-    candidate(matrix_, 3, &matrix, xy_matrix);
+    candidate(mayMatrix, 3, &matrix, xy_matrix);
   };
   if (forward) {
     time_xy();
@@ -743,7 +747,7 @@ void ExecutionGPU<T>::download(char* dst, const char* src, size_t bytes, size_t 
 }
 
 template <typename T>
-void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent) {
+void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent, Families families) {
   hipStream_t stream = begin(concurrent);
   // copies go to the transform's own stream, beside the kernels on the
   // default stream (batched fallbacks run both on the transform's stream)
@@ -774,13 +778,16 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent) {
   }
   T* outGPU = hostOut ? grid_->space_gpu() : outView;
   hipEvent_t* ready = &ioEvents_[0];
+  // of the FFT kernels, lengths that are not fixed have the generic ones only
+  const bool fast = fast_ && (families == Families::kAll || tab_->fixedLengths);
+  if (!fast && !tab_->generic) throw InternalError();
 
-  if (fast_) {
+  if (fast) {
     FastArgs<T> f = fast_args();
     f.in = inGPU;
     f.out = outGPU;
     const TuneChoice choice =
-        single_choice(false, f, stream, inKind != MemKind::Device || hostOut);
+        single_choice(false, f, stream, inKind != MemKind::Device || hostOut, families);
     const int fromValues = choice.plane == 3 ? from_values(false) : 0;
     if (fromValues == 0) {
       f.hasRuns = choice.zRuns;
@@ -1185,7 +1192,8 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
 template <typename T>
 bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
                                 const std::vector<const T*>& in, const std::vector<T*>& out,
-                                bool forward, const std::vector<SpfftScalingType>& scaling) {
+                                bool forward, const std::vector<SpfftScalingType>& scaling,
+                                Families families) {
   const size_t n = ex.size();
   if (n < 2) return false;
   std::vector<const T*> din(n);
@@ -1194,6 +1202,14 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   if (!batch_qualifies(ex.data(), n, in.data(), out.data(), din.data(), dout.data(), &shape)) {
     return false;
   }
+  const bool fft = families == Families::kFft;
+  if (fft && !shape.fixedLengths) {
+    // one after the other on the default stream (the generic kernels)
+    for (size_t t = 0; t < n; ++t) ex[t]->backward(din[t], dout[t], false, families);
+    return true;
+  }
+  shape.matrix = shape.matrix && !fft;
+  shape.fromValues = shape.fromValues && !fft;
   const int nt = static_cast<int>(n);
 
   std::vector<std::uint64_t> key;
@@ -1262,7 +1278,7 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
     choice.plane = 3;  // nothing to choose
   } else {
     const TuneKey tkey = make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
-                                       shape.dimY, shape.dimZ, shape.r2c, forward,
+                                       shape.dimY, shape.dimZ, shape.r2c, forward, fft,
                                        shape.maxNcol, shape.maxNst, nt);
     if (!tune_lookup(tkey, &choice)) {
       choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap);
@@ -1315,8 +1331,8 @@ void ExecutionGPU<T>::run_batch_noalloc(ExecutionGPU<T>* const* ex, size_t n, co
     choice.plane = forced;
   } else {
     (void)tune_recorded(make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
-                                      shape.dimY, shape.dimZ, shape.r2c, forward, shape.maxNcol,
-                                      shape.maxNst, static_cast<int>(n)),
+                                      shape.dimY, shape.dimZ, shape.r2c, forward, false,
+                                      shape.maxNcol, shape.maxNst, static_cast<int>(n)),
                         &choice);
   }
   if (choice.plane == 1 && !plane_candidate(ex, n, din, dout, forward, shape)) {

@@ -20,6 +20,10 @@
 
 namespace spfft {
 
+// Kernel families that a call may use. kFft leaves out the matrix kernels: FP32
+// fields then carry the rounding of FFT passes, whatever lengths they have.
+enum class Families { kAll, kFft };
+
 // Device index tables and twiddles of one index set on one device. Built once
 // and shared by every transform with an identical set (same dimensions, type,
 // precision and value order), so the bands of one set hold, and a batch of
@@ -30,6 +34,7 @@ struct TransformTables {
   int device = 0;
   bool allowFast = true;  // built with the fixed-length path allowed
   bool fast = false;      // fixed-length or matrix kernels serve this set
+  bool generic = false;   // the generic kernels' tables are here
   bool split = false;     // the split plane stage does (fixed Nx and Ny)
   bool matrix = false;    // the matrix plane kernels do
   bool classSplit = false;    // the class-split plane kernels do (nx = ny, LDS fits)
@@ -63,7 +68,8 @@ public:
   // 403-410) without cross-stream hops. Batched calls (concurrent = true) run
   // on the transform's own stream, fenced against the default stream with
   // events, so independent transforms overlap.
-  void backward(const T* input, T* output, bool concurrent = false);
+  void backward(const T* input, T* output, bool concurrent = false,
+                Families families = Families::kAll);
   void forward(const T* input, T* output, SpfftScalingType scaling, bool concurrent = false);
   // SYNCHRONOUS: wait for the work. ASYNCHRONOUS: return; a concurrent call
   // additionally makes the default stream wait for its stream.
@@ -77,7 +83,8 @@ public:
   // not qualify (different shapes, generic lengths, host pointers, empty sets).
   static bool run_batch(const std::vector<ExecutionGPU<T>*>& ex, const std::vector<const T*>& in,
                         const std::vector<T*>& out, bool forward,
-                        const std::vector<SpfftScalingType>& scaling);
+                        const std::vector<SpfftScalingType>& scaling,
+                        Families families = Families::kAll);
 
   // Pieces of the fused batch, shared by run_batch and the allocation-free
   // batched entry point (which keeps its tables in a static device array).
@@ -175,7 +182,8 @@ private:
   // matrix kernels; z addressing when the sticks are runs), tuned on the first call
   // of the shape with device input and output, on that call's buffers
   // (staged = host data in the work buffer: recorded choices or defaults).
-  TuneChoice single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream, bool staged);
+  TuneChoice single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream, bool staged,
+                           Families families = Families::kAll);
 
   std::shared_ptr<IndexMap> map_;
   std::shared_ptr<GridInternal<T>> grid_;

@@ -29,6 +29,15 @@ __device__ __forceinline__ double block_sum(double x) {
   return x;
 }
 
+// |x|^2. An FP32 field is squared in FP32, operation by operation: the energy is
+// the FP64 sum of the FP32 density sum V rho, whatever computes the density.
+__device__ __forceinline__ double density(Cx<double> x) { return x.re * x.re + x.im * x.im; }
+__device__ __forceinline__ double density(Cx<float> x) {
+#pragma clang fp contract(off)
+  const float re = x.re * x.re, im = x.im * x.im;
+  return static_cast<double>(re + im);
+}
+
 // partial[band][block] = the block's share of sum_r V |psi|^2, in FP64.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
@@ -51,8 +60,7 @@ __global__ void __launch_bounds__(kThreads)
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const double re = x[u].re, im = x[u].im;
-      acc += static_cast<double>(w[u]) * (re * re + im * im);
+      acc += static_cast<double>(w[u]) * density(x[u]);
     }
   }
   acc = block_sum(acc);

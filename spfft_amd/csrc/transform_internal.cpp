@@ -100,14 +100,14 @@ void TransformInternal<T>::forward_enqueue(const T* input, T* output, SpfftScali
 }
 
 template <typename T>
-void TransformInternal<T>::backward_enqueue(const T* input, T* output) {
+void TransformInternal<T>::backward_enqueue(const T* input, T* output, Families families) {
   if (execHost_) {
     execHost_->backward(input, output);
     return;
   }
   check_preceding();
   DeviceGuard guard(grid_->device_id());
-  exec_->backward(input, output, true);
+  exec_->backward(input, output, true, families);
 }
 
 template <typename T>
@@ -122,11 +122,12 @@ template <typename T>
 bool run_batched(const std::vector<TransformInternal<T>*>& ts,
                  const std::vector<std::shared_ptr<ExecutionGPU<T>>>& execs,
                  const std::vector<const T*>& in, const std::vector<T*>& out, bool forward,
-                 const std::vector<SpfftScalingType>& scaling, int device) {
+                 const std::vector<SpfftScalingType>& scaling, int device,
+                 Families families = Families::kAll) {
   std::vector<ExecutionGPU<T>*> ex;
   for (const auto& e : execs) ex.push_back(e.get());
   DeviceGuard guard(device);
-  if (!ExecutionGPU<T>::run_batch(ex, in, out, forward, scaling)) return false;
+  if (!ExecutionGPU<T>::run_batch(ex, in, out, forward, scaling, families)) return false;
   bool sync = false;
   for (const TransformInternal<T>* t : ts) sync |= t->execution_mode() == SPFFT_EXEC_SYNCHRONOUS;
   if (sync) check_hip(hipStreamSynchronize(nullptr));
@@ -137,7 +138,7 @@ bool run_batched(const std::vector<TransformInternal<T>*>& ts,
 template <typename T>
 bool TransformInternal<T>::batch_backward(const std::vector<TransformInternal*>& ts,
                                           const std::vector<const T*>& in,
-                                          const std::vector<T*>& out) {
+                                          const std::vector<T*>& out, Families families) {
   if (ts.empty()) return false;
   for (TransformInternal* t : ts) {
     if (!t->exec_) return false;  // host transforms run one by one
@@ -145,7 +146,7 @@ bool TransformInternal<T>::batch_backward(const std::vector<TransformInternal*>&
   check_preceding();
   std::vector<std::shared_ptr<ExecutionGPU<T>>> execs;
   for (TransformInternal* t : ts) execs.push_back(t->exec_);
-  return run_batched<T>(ts, execs, in, out, false, {}, ts[0]->device_id());
+  return run_batched<T>(ts, execs, in, out, false, {}, ts[0]->device_id(), families);
 }
 
 template <typename T>

@@ -30,13 +30,14 @@ public:
 
   // Enqueue without the final synchronisation (batched execution).
   void forward_enqueue(const T* input, T* output, SpfftScalingType scaling);
-  void backward_enqueue(const T* input, T* output);
+  void backward_enqueue(const T* input, T* output, Families families = Families::kAll);
   void synchronize();
 
   // One fused launch chain for a batch of transforms of one shape (see
   // ExecutionGPU::run_batch); false when the batch does not qualify.
   static bool batch_backward(const std::vector<TransformInternal*>& ts,
-                             const std::vector<const T*>& in, const std::vector<T*>& out);
+                             const std::vector<const T*>& in, const std::vector<T*>& out,
+                             Families families = Families::kAll);
   static bool batch_forward(const std::vector<TransformInternal*>& ts,
                             const std::vector<const T*>& in, const std::vector<T*>& out,
                             const std::vector<SpfftScalingType>& scaling);

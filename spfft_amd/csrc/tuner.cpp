@@ -4,6 +4,7 @@
 #include <sys/stat.h>
 #include <unistd.h>
 
+#include <array>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -11,11 +12,12 @@
 #include <mutex>
 #include <sstream>
 #include <string>
-#include <tuple>
 
 namespace spfft {
 
 namespace {
+
+using NumericKey = std::array<int, 11>;
 
 struct TuneState {
   std::mutex mutex;
@@ -24,12 +26,12 @@ struct TuneState {
   std::map<std::string, TuneChoice> choices;
   std::map<int, std::string> arch;  // device -> "gfx950:256"
   // choices this process has used, by numeric key
-  std::map<std::tuple<int, int, int, int, int, int, int, int, int, int>, TuneChoice> used;
+  std::map<NumericKey, TuneChoice> used;
 };
 
-std::tuple<int, int, int, int, int, int, int, int, int, int> numeric(const TuneKey& k) {
-  return std::make_tuple(k.device, k.valueBytes, k.n, k.ny, k.nz, k.r2c, k.forward, k.ncolBucket,
-                         k.stickBucket, k.countBucket);
+NumericKey numeric(const TuneKey& k) {
+  return {k.device,  k.valueBytes, k.n,          k.ny,          k.nz,         k.r2c,
+          k.forward, k.fft,        k.ncolBucket, k.stickBucket, k.countBucket};
 }
 
 TuneState& state() {
@@ -118,7 +120,7 @@ int round_quarter(int v) {
 }  // namespace
 
 TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2c, bool forward,
-                      int maxNcol, int maxNst, int count) {
+                      bool fft, int maxNcol, int maxNst, int count) {
   TuneKey k;
   k.device = device;
   k.valueBytes = valueBytes;
@@ -127,6 +129,7 @@ TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2
   k.nz = nz;
   k.r2c = r2c ? 1 : 0;
   k.forward = forward ? 1 : 0;
+  k.fft = fft ? 1 : 0;
   k.ncolBucket = (maxNcol + 15) / 16 * 16;
   k.stickBucket = round_quarter(maxNst);
   k.countBucket = round_pow2(count < 1 ? 1 : count);
@@ -159,7 +162,7 @@ std::string tune_key_text(const TuneKey& k) {
   o << arch << ":f" << 8 * k.valueBytes << ":N" << k.n;
   if (k.ny != k.n) o << "x" << k.ny;
   o << ":Z" << k.nz << ":"
-    << (k.r2c ? "r2c" : "c2c") << ":" << (k.forward ? "fwd" : "bwd") << ":col" << k.ncolBucket
+    << (k.r2c ? "r2c" : "c2c") << ":" << (k.forward ? "fwd" : "bwd") << (k.fft ? ":fft" : "") << ":col" << k.ncolBucket
     << ":st" << k.stickBucket << ":x" << k.countBucket;
   return o.str();
 }

@@ -3,7 +3,7 @@
 // per-shape cache file, so later processes start from the measured choices.
 //
 // Key: device architecture and CU count, value bytes, Nx, Ny, Nz, C2C or R2C,
-// direction, widest column count (rounded up to 16), most sticks (rounded up to
+// direction, whether the matrix kernels may run, widest column count (rounded up to 16), most sticks (rounded up to
 // a quarter of an octave, since the work of a plane follows them) and transform
 // count (rounded up to a power of two; 1 for single transforms).
 // Choices: the plane-kernel family of batches (class-split kernels with R
@@ -29,6 +29,7 @@ struct TuneKey {
   int valueBytes = 0;
   int n = 0, ny = 0, nz = 0;
   int r2c = 0, forward = 0;
+  int fft = 0;  // without the matrix kernels
   int ncolBucket = 0, stickBucket = 0, countBucket = 0;
 };
 
@@ -41,7 +42,7 @@ struct TuneChoice {
 };
 
 TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2c, bool forward,
-                      int maxNcol, int maxNst, int count);
+                      bool fft, int maxNcol, int maxNst, int count);
 // The recorded choice for `key` (from this process or the cache file).
 bool tune_lookup(const TuneKey& key, TuneChoice* choice);
 // Records a timed choice and rewrites the cache file.
