@@ -125,6 +125,12 @@ int served_plane(int want, bool classSplit, bool split, bool matrix) {
   return classSplit ? 0 : (split ? 2 : 3);
 }
 
+bool overlap(const void* a, size_t aBytes, const void* b, size_t bBytes) {
+  const char* pa = static_cast<const char*>(a);
+  const char* pb = static_cast<const char*>(b);
+  return pa < pb + bBytes && pb < pa + aBytes;
+}
+
 // Mean time of `reps` launches after one warm-up launch, in milliseconds.
 template <typename F>
 float time_launches(F&& launch, hipEvent_t e0, hipEvent_t e1, int reps = 3) {
@@ -163,6 +169,7 @@ std::atomic<std::uint64_t> next_serial{1};
 // launches, and 300 us to make.
 struct BatchPlan {
   std::vector<std::uint64_t> key;
+  bool inPlace = false;  // an input overlaps an output
   int device = 0;
   void* args = nullptr;
   void* map = nullptr;
@@ -788,7 +795,10 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent, Famil
     f.out = outGPU;
     const TuneChoice choice =
         single_choice(false, f, stream, inKind != MemKind::Device || hostOut, families);
-    const int fromValues = choice.plane == 3 ? from_values(false) : 0;
+    // Values that lie in the field are all read before its first plane is written.
+    const bool inPlace =
+        overlap(inGPU, valueBytes, outGPU, space_domain_size() * sizeof(T));
+    const int fromValues = choice.plane == 3 && !inPlace ? from_values(false) : 0;
     if (fromValues == 0) {
       f.hasRuns = choice.zRuns;
       launch_z<T>(false, map_->dimX, map_->dimY, map_->dimZ, f, stream);
@@ -1001,6 +1011,21 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
                       dft_values_supported<T>(shape->r2c, m0.dimX, m0.dimY, m0.dimZ, shape->kx,
                                               shape->ky);
   return shape->split || shape->matrix;
+}
+
+template <typename T>
+bool ExecutionGPU<T>::batch_in_place(ExecutionGPU<T>* const* ex, size_t n, const T* const* din,
+                                     T* const* dout, bool forward) {
+  auto bytes = [&](size_t t, bool space) {
+    return sizeof(T) * (space ? ex[t]->space_domain_size()
+                              : 2 * static_cast<size_t>(ex[t]->map_->num_values()));
+  };
+  for (size_t t = 0; t < n; ++t) {
+    for (size_t u = 0; u < n; ++u) {
+      if (overlap(din[t], bytes(t, forward), dout[u], bytes(u, !forward))) return true;
+    }
+  }
+  return false;
 }
 
 template <typename T>
@@ -1258,6 +1283,7 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
     launch_batch_tables<T>(args.data(), nt, sticks_per_block<T>(shape.dimZ),
                            static_cast<FastArgs<T>*>(plan.args), static_cast<int2*>(plan.map),
                            nullptr);
+    plan.inPlace = batch_in_place(ex.data(), n, din.data(), dout.data(), forward);
     plan.key = std::move(key);
     hit = cache.plans.begin();
   } else if (hit != cache.plans.begin()) {
@@ -1267,6 +1293,7 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   BatchPlan& plan = *hit;
   const auto* dArgs = static_cast<const FastArgs<T>*>(plan.args);
   const auto* dMap = static_cast<const int2*>(plan.map);
+  shape.fromValues = shape.fromValues && !plan.inPlace;
 
   // kernel choices: forced plane family, recorded (this process or the cache
   // file), or timed now on this batch's buffers
@@ -1313,6 +1340,7 @@ void ExecutionGPU<T>::run_batch_noalloc(ExecutionGPU<T>* const* ex, size_t n, co
   if (!batch_qualifies(ex, n, in, out, din, dout, &shape) || !shape.fixedLengths) {
     throw InvalidParameterError();
   }
+  shape.fromValues = shape.fromValues && !forward && !batch_in_place(ex, n, din, dout, false);
   const size_t argBytes = (n * sizeof(FastArgs<T>) + 255) / 256 * 256;
   const size_t tableBytes = argBytes + static_cast<size_t>(shape.blocks) * sizeof(int2);
   if (tableBytes > scratchBytes || viewBytes + tableBytes > stageBytes) {

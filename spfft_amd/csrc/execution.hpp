@@ -106,6 +106,9 @@ public:
   // entries each) hold the device views of the user pointers.
   static bool batch_qualifies(ExecutionGPU* const* ex, size_t n, const T* const* in,
                               T* const* out, const T** din, T** dout, BatchShape* shape);
+  // True when an input of the batch overlaps an output (its own or another's).
+  static bool batch_in_place(ExecutionGPU* const* ex, size_t n, const T* const* din,
+                             T* const* dout, bool forward);
   // True when the whole-plane kernels can serve the batch.
   static bool plane_candidate(ExecutionGPU* const* ex, size_t n, const T* const* din,
                               T* const* dout, bool forward, const BatchShape& shape);
