@@ -556,7 +556,7 @@ FastArgs<T> ExecutionGPU<T>::fast_args() const {
 
 template <typename T>
 TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream,
-                                          bool staged, Families families) {
+                                          bool keepInput, Families families) {
   TuneChoice c;
   c.zRuns = f.hasRuns;
   const int forced = plane_kernels_forced();
@@ -581,10 +581,11 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     c.plane = served_plane(known.plane, classSplit_, split_, mayMatrix);
     return c;
   }
-  // Host data staged in the work buffer, which the split stage's candidate
-  // launches would overwrite: no timing on this call (defaults).
-  if (staged) return c;
-  // Every launch below is idempotent: backward z reads the values and writes
+  // Timing would overwrite host data staged in the work buffer (by the split
+  // stage's column buffer) and an input that shares memory with the output: no
+  // timing on such a call (defaults).
+  if (keepInput) return c;
+  // Every launch below is idempotent, its input and output apart: backward z reads the values and writes
   // the [z][stick] buffer, the plane stage reads that buffer and writes the
   // output; forward the plane stage reads the input and writes the buffer,
   // z reads it and writes the values. The call's real launches follow.
@@ -793,11 +794,11 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent, Famil
     FastArgs<T> f = fast_args();
     f.in = inGPU;
     f.out = outGPU;
-    const TuneChoice choice =
-        single_choice(false, f, stream, inKind != MemKind::Device || hostOut, families);
-    // Values that lie in the field are all read before its first plane is written.
     const bool inPlace =
         overlap(inGPU, valueBytes, outGPU, space_domain_size() * sizeof(T));
+    const TuneChoice choice = single_choice(
+        false, f, stream, inKind != MemKind::Device || hostOut || inPlace, families);
+    // Values that lie in the field are all read before its first plane is written.
     const int fromValues = choice.plane == 3 && !inPlace ? from_values(false) : 0;
     if (fromValues == 0) {
       f.hasRuns = choice.zRuns;
@@ -889,7 +890,8 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
     f.out = outGPU;
     f.useScale = scaling == SPFFT_FULL_SCALING ? 1 : 0;
     const TuneChoice choice =
-        single_choice(true, f, stream, hostIn || outKind != MemKind::Device);
+        single_choice(true, f, stream, hostIn || outKind != MemKind::Device ||
+                                           overlap(inGPU, spaceBytes, outGPU, valueBytes));
     // host input: each chunk of planes is transformed as soon as it arrives
     for (int c = 0; c < chunks; ++c) {
       if (hostIn) upload_chunk(c);
@@ -1307,7 +1309,8 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
     const TuneKey tkey = make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
                                        shape.dimY, shape.dimZ, shape.r2c, forward, fft,
                                        shape.maxNcol, shape.maxNst, nt);
-    if (!tune_lookup(tkey, &choice)) {
+    // (timing would overwrite inputs that share memory with outputs)
+    if (!tune_lookup(tkey, &choice) && !plan.inPlace) {
       choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap);
       tune_record(tkey, choice);
     }

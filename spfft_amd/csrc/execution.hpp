@@ -184,8 +184,8 @@ private:
   // Kernel choices of a single transform (plane stage: class-split, split or
   // matrix kernels; z addressing when the sticks are runs), tuned on the first call
   // of the shape with device input and output, on that call's buffers
-  // (staged = host data in the work buffer: recorded choices or defaults).
-  TuneChoice single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream, bool staged,
+  // (keepInput = timing would overwrite the input: recorded choices or defaults).
+  TuneChoice single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream, bool keepInput,
                            Families families = Families::kAll);
 
   std::shared_ptr<IndexMap> map_;
