@@ -37,9 +37,9 @@ import spfft_amd as sp
 _i, _ll, _vp = ctypes.c_int, ctypes.c_longlong, ctypes.c_void_p
 sp.lib.spfft_amd_energy_partials.argtypes = [_i]
 sp.lib.spfft_amd_energy_partials.restype = _i
-sp.lib.spfft_amd_field_energy.argtypes = [_i, _vp, _vp, _ll, _i, _vp, _vp, _vp]
+sp.lib.spfft_amd_field_energy.argtypes = [_i, _i, _vp, _vp, _ll, _i, _vp, _vp, _vp]
 sp.lib.spfft_amd_field_energy.restype = _i
-sp.lib.spfft_amd_energy_field.argtypes = [_i, _vp, _vp, _vp, _ll, _i, _vp, _vp]
+sp.lib.spfft_amd_energy_field.argtypes = [_i, _i, _vp, _vp, _vp, _ll, _i, _vp, _vp]
 sp.lib.spfft_amd_energy_field.restype = _i
 sp.lib.spfft_amd_float_backward_fft.argtypes = [_i] + 3 * [ctypes.POINTER(_vp)]
 sp.lib.spfft_amd_float_backward_fft.restype = _i
@@ -72,11 +72,15 @@ def _check_transform(transform, dims):
 
 
 class _OnDefaultStream:
-    """Orders a library call (HIP default stream) against torch's current stream."""
+    """Orders a library call (the HIP default stream of `device`, whichever device is
+    current) against torch's current stream there."""
+
+    def __init__(self, device):
+        self.device = device
 
     def __enter__(self):
-        self.cur = torch.cuda.current_stream()
-        self.dflt = torch.cuda.default_stream()
+        self.cur = torch.cuda.current_stream(self.device)
+        self.dflt = torch.cuda.default_stream(self.device)
         self.other = self.cur.cuda_stream != self.dflt.cuda_stream
         if self.other:
             self.dflt.wait_stream(self.cur)
@@ -93,7 +97,7 @@ def _backward(transform, dims, c):
     _check_tensor("c", c, transform, transform.num_values)
     c = c.contiguous()
     psi = torch.empty((nz, ny, nx), dtype=c.dtype, device=c.device)
-    with _OnDefaultStream():
+    with _OnDefaultStream(c.device):
         transform.backward(torch.view_as_real(c).data_ptr(), torch.view_as_real(psi).data_ptr())
     return psi
 
@@ -104,7 +108,7 @@ def _adjoint(transform, n, field):
                   transform.dim_x() * transform.dim_y() * transform.dim_z())
     field = field.contiguous()
     out = torch.empty(n, dtype=field.dtype, device=field.device)
-    with _OnDefaultStream():
+    with _OnDefaultStream(field.device):
         transform.forward(torch.view_as_real(field).data_ptr(),
                           torch.view_as_real(out).data_ptr(), sp.SPFFT_NO_SCALING)
     return out
@@ -153,10 +157,10 @@ def sparse_energy(c, potential, transform, dims, recompute=True):
     return SparseEnergy.apply(c, potential, transform, dims, recompute)
 
 
-def _field_budget(memory_budget):
+def _field_budget(memory_budget, device=None):
     if memory_budget is not None:
         return int(memory_budget)
-    free, _ = torch.cuda.mem_get_info()
+    free, _ = torch.cuda.mem_get_info(device)
     return free // 4
 
 
@@ -189,7 +193,7 @@ def _batch_backward(transforms, dims, C, for_energy=False):
     _check_tensor("C", C, transforms[0], len(transforms) * n)
     C = C.contiguous()
     psi = torch.empty((len(transforms), nz, ny, nx), dtype=C.dtype, device=C.device)
-    with _OnDefaultStream():
+    with _OnDefaultStream(C.device):
         if for_energy and C.dtype == torch.complex64:
             _float_backward_fft(transforms, _rows(C), _rows(psi))
         else:
@@ -200,19 +204,19 @@ def _batch_backward(transforms, dims, C, for_energy=False):
 def _batch_adjoint(transforms, n, fields):
     out = torch.empty((len(transforms), n), dtype=fields.dtype, device=fields.device)
     fields = fields.contiguous()
-    with _OnDefaultStream():
+    with _OnDefaultStream(fields.device):
         sp.multi_transform_forward(transforms, _rows(fields), _rows(out),
                                    [sp.SPFFT_NO_SCALING] * len(transforms))
     return out
 
 
-def recompute_fields(field_bytes, recompute="auto", memory_budget=None):
+def recompute_fields(field_bytes, recompute="auto", memory_budget=None, device=None):
     """True when the batched energy's backward recomputes the fields: always
     for recompute=True, never for False, and for "auto" when the fields
     (field_bytes) exceed the budget (memory_budget bytes, or a quarter of the
-    device memory free now)."""
+    memory free now on `device`, the current one if None)."""
     if recompute == "auto":
-        return field_bytes > _field_budget(memory_budget)
+        return field_bytes > _field_budget(memory_budget, device)
     return bool(recompute)
 
 
@@ -236,9 +240,9 @@ def _band_energy(psi, potential):
                           device=psi.device)
     energy = torch.empty((), dtype=torch.float64, device=psi.device)
     sp._check(sp.lib.spfft_amd_field_energy(
-        potential.element_size(), psi.data_ptr(), potential.data_ptr(), potential.numel(), bands,
-        partial.data_ptr(), energy.data_ptr(), torch.cuda.current_stream().cuda_stream),
-        "field_energy")
+        psi.device.index, potential.element_size(), psi.data_ptr(), potential.data_ptr(),
+        potential.numel(), bands, partial.data_ptr(), energy.data_ptr(),
+        torch.cuda.current_stream(psi.device).cuda_stream), "field_energy")
     return energy
 
 
@@ -257,9 +261,9 @@ def _energy_gradient(transforms, psi, own, potential, grad_energy):
              not grad_energy.is_neg() else None)
     field = psi if own else torch.empty_like(psi)
     sp._check(sp.lib.spfft_amd_energy_field(
-        potential.element_size(), psi.data_ptr(), potential.data_ptr(),
+        psi.device.index, potential.element_size(), psi.data_ptr(), potential.data_ptr(),
         None if scale is None else scale.data_ptr(), potential.numel(), psi.shape[0],
-        field.data_ptr(), torch.cuda.current_stream().cuda_stream), "energy_field")
+        field.data_ptr(), torch.cuda.current_stream(psi.device).cuda_stream), "energy_field")
     g = _batch_adjoint(transforms, n, field)
     return g if scale is not None else grad_energy.to(potential.dtype) * g
 
@@ -271,7 +275,7 @@ class SparseEnergyBatch(torch.autograd.Function):
         energy = _band_energy(psi, potential)
         ctx.transforms, ctx.dims = transforms, dims
         ctx.recompute = recompute_fields(psi.numel() * psi.element_size(), recompute,
-                                         memory_budget)
+                                         memory_budget, psi.device)
         if ctx.recompute:
             ctx.save_for_backward(C, potential)
         else:

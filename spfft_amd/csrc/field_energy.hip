@@ -135,18 +135,19 @@ int guarded(F&& f) {
 }  // namespace spfft
 
 // Hooks of spfft_amd/autograd.py (no counterpart in the reference ABI): device
-// pointers of checked tensors, `stream` the caller's. valueBytes: 8 or 4 per real
+// pointers of checked tensors on `device`, `stream` the caller's there. valueBytes: 8 or 4 per real
 // value. `partial` holds spfft_amd_energy_partials(bands) doubles.
 extern "C" __attribute__((visibility("default"))) int spfft_amd_energy_partials(int bands) {
   return spfft::kEnergyBlocks * bands;
 }
 extern "C" __attribute__((visibility("default"))) int spfft_amd_field_energy(
-    int valueBytes, const void* psi, const void* potential, long long points, int bands,
-    double* partial, double* energy, void* stream) {
+    int device, int valueBytes, const void* psi, const void* potential, long long points,
+    int bands, double* partial, double* energy, void* stream) {
   using namespace spfft;
   const auto s = static_cast<hipStream_t>(stream);
   return guarded([&] {
     if (points < 1 || bands < 1 || bands > 65535) throw InvalidParameterError();
+    DeviceGuard guard(device);
     if (valueBytes == 8) {
       field_energy<double>(psi, potential, points, bands, partial, energy, s);
     } else {
@@ -155,12 +156,13 @@ extern "C" __attribute__((visibility("default"))) int spfft_amd_field_energy(
   });
 }
 extern "C" __attribute__((visibility("default"))) int spfft_amd_energy_field(
-    int valueBytes, const void* psi, const void* potential, const double* grad, long long points,
-    int bands, void* out, void* stream) {
+    int device, int valueBytes, const void* psi, const void* potential, const double* grad,
+    long long points, int bands, void* out, void* stream) {
   using namespace spfft;
   const auto s = static_cast<hipStream_t>(stream);
   return guarded([&] {
     if (points < 1 || bands < 1 || bands > 65535) throw InvalidParameterError();
+    DeviceGuard guard(device);
     if (valueBytes == 8) {
       energy_field<double>(psi, potential, grad, points, bands, out, s);
     } else {
