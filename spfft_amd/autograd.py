@@ -246,6 +246,14 @@ def _band_energy(psi, potential):
     return energy
 
 
+def _address(x):
+    """The address of x; None for one of vmap's, which has no memory of its own."""
+    try:
+        return x.data_ptr()
+    except RuntimeError:
+        return None
+
+
 def _energy_gradient(transforms, psi, own, potential, grad_energy):
     """grad_energy * 2 B^H (V psi) per band. own: psi belongs to the call, so the
     field may take its place."""
@@ -256,14 +264,13 @@ def _energy_gradient(transforms, psi, own, potential, grad_energy):
         return grad_energy.to(potential.dtype) * g
     # FP64: the factor goes into the field; FP32: its product with the potential
     # could leave float32's range where the gradient does not
-    scale = (grad_energy if potential.dtype == torch.float64 and
+    scale = (_address(grad_energy) if potential.dtype == torch.float64 and
              grad_energy.dtype == torch.float64 and grad_energy.device == psi.device and
              not grad_energy.is_neg() else None)
     field = psi if own else torch.empty_like(psi)
     sp._check(sp.lib.spfft_amd_energy_field(
-        psi.device.index, potential.element_size(), psi.data_ptr(), potential.data_ptr(),
-        None if scale is None else scale.data_ptr(), potential.numel(), psi.shape[0],
-        field.data_ptr(), torch.cuda.current_stream(psi.device).cuda_stream), "energy_field")
+        psi.device.index, potential.element_size(), psi.data_ptr(), potential.data_ptr(), scale,
+        potential.numel(), psi.shape[0], field.data_ptr(), torch.cuda.current_stream(psi.device).cuda_stream), "energy_field")
     g = _batch_adjoint(transforms, n, field)
     return g if scale is not None else grad_energy.to(potential.dtype) * g
 
