@@ -117,9 +117,33 @@ void launch_z(bool forward, int nx, int ny, int nz, const FastArgs<T>& a, hipStr
 // 9.6 / 10.2; batches of 8: 28^3 11.6 / 9.8, 36^3 13.2 / 18.7.
 constexpr int kFromValues = 3000;
 
+// True when the generic kernels may beat the matrix kernels on a set that is not
+// all of fixed lengths: long lines and no prime factor that they sum directly.
+// Pairs, generic / matrix kernels, us, spheres of radius 0.24, 0.30 and 0.47 N:
+//   245^3 FP64 503 / 403, 633 / 700, 1066 / 1319; FP32 380 / 339, 440 / 476, 725 / 943
+//   250^3 FP64 634 / 381, 761 / 748, 1262 / 1305; FP32 447 / 249, 537 / 446, 858 / 734
+//   308^3 FP64 1068 / 1134, 1307 / 1294, 2152 / 2972; R2C FP64 782 / 676, 909 / 770,
+//     1331 / 1886
+// (the matrix kernels' work follows the square of the radius). Shorter lines all run
+// faster on the matrix kernels or even (radius 0.47 N: 143^3 FP64 199 / 184, FP32 174 /
+// 178; 143 x 160 x 160 257 / 228, 206 / 191), and so do sets with a prime factor above
+// 13 (1.5 times at 17 x 320 x 320, radius 0.47 N; 2.6 to 47 at 221^3 to 319^3).
+bool generic_candidate(int nx, int ny, int nz) {
+  auto smooth = [](int n) {
+    for (int p : {2, 3, 5, 7, 11, 13}) {
+      while (n % p == 0) n /= p;
+    }
+    return n == 1;
+  };
+  return std::max({nx, ny, nz}) > 160 && smooth(nx) && smooth(ny) && smooth(nz);
+}
+
 // The plane family to run for `want` among those that serve the shape: the
-// class-split kernels, else the split stage, else the matrix kernels.
-int served_plane(int want, bool classSplit, bool split, bool matrix) {
+// class-split kernels, else the split stage, else the matrix kernels (or the generic
+// kernels for all stages, where they are a candidate).
+constexpr int kGenericKernels = 4;
+int served_plane(int want, bool classSplit, bool split, bool matrix, bool generic = false) {
+  if (want == kGenericKernels && generic) return kGenericKernels;
   if (want == 3 && matrix) return 3;
   if (want == 2 && split) return 2;
   return classSplit ? 0 : (split ? 2 : 3);
@@ -236,7 +260,9 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
   // each set's tables are those that its kernels read
   tb.stickBegin = DeviceBuffer<int>::from_host(t.stickBegin);
   // The energy of FP32 bands takes its fields from FFT kernels (Families::kFft).
-  tb.generic = !useFast || (sizeof(T) == 4 && !r2c && !tb.fixedLengths);
+  tb.tryGeneric = useFast && !tb.fixedLengths &&
+                  generic_candidate(map->dimX, map->dimY, map->dimZ);
+  tb.generic = !useFast || tb.tryGeneric || (sizeof(T) == 4 && !r2c && !tb.fixedLengths);
   if (tb.generic) {
     tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
     tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
@@ -555,6 +581,34 @@ FastArgs<T> ExecutionGPU<T>::fast_args() const {
 }
 
 template <typename T>
+void ExecutionGPU<T>::launch_generic(bool forward, const T* in, T* out, bool useScale,
+                                     hipStream_t stream) {
+  if (!tab_->generic) throw InternalError();
+  StageArgs<T> a = base_args();
+  a.in = in;
+  a.out = out;
+  a.useScale = useScale ? 1 : 0;
+  auto stage = [&](const FftDesc& fft, const DeviceBuffer<Tw<T>>& tw, int batch,
+                   void (*launch)(const StageArgs<T>&, hipStream_t)) {
+    a.fft = fft;
+    a.tw = tw.data();
+    a.batch = batch;
+    launch(a, stream);
+  };
+  if (forward) {
+    stage(fftX_, tab_->twX, xBatch_, launch_x_forward<T>);
+    stage(fftY_, tab_->twY, yBatch_, launch_y_forward<T>);
+    stage(fftZ_, tab_->twZ, zBatch_, launch_z_forward<T>);
+  } else {
+    if (a.nst > 0) {
+      stage(fftZ_, tab_->twZ, zBatch_, launch_z_backward<T>);
+      stage(fftY_, tab_->twY, yBatch_, launch_y_backward<T>);
+    }
+    stage(fftX_, tab_->twX, xBatch_, launch_x_backward<T>);
+  }
+}
+
+template <typename T>
 TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hipStream_t stream,
                                           bool keepInput, Families families) {
   TuneChoice c;
@@ -567,18 +621,19 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   // lengths that are not fixed only the latter
   c.plane = served_plane(forced, classSplit_, split_, mayMatrix);
   if (forced >= 0) return c;
+  const bool tryGeneric = tab_->tryGeneric && !fft;
   // batched fallbacks on the transform's own stream keep the defaults
   if (stream != nullptr) return c;
   const bool fixedZ = fixed_length(map_->dimZ);
   // nothing to choose
-  if (!split_ && !(fixedZ && f.hasRuns)) return c;
+  if (!split_ && !(fixedZ && f.hasRuns) && !tryGeneric) return c;
   const TuneKey key = make_tune_key(grid_->device_id(), static_cast<int>(sizeof(T)), map_->dimX,
                                     map_->dimY, map_->dimZ, map_->type == SPFFT_TRANS_R2C,
                                     forward, fft, numCols_, map_->num_sticks(), 1);
   TuneChoice known;
   if (tune_lookup(key, &known)) {
     c.zRuns = known.zRuns && f.hasRuns;
-    c.plane = served_plane(known.plane, classSplit_, split_, mayMatrix);
+    c.plane = served_plane(known.plane, classSplit_, split_, mayMatrix, tryGeneric);
     return c;
   }
   // Timing would overwrite host data staged in the work buffer (by the split
@@ -612,13 +667,13 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     a.hasRuns = f.hasRuns;
     launch_dft_xy<T>(forward, map_->dimX, map_->dimY, fromValues, a, nullptr);
   };
-  float zr = 0.f, ze = 0.f, fused = 0.f, two = 0.f, matrix = 0.f;
+  float zr = 0.f, ze = 0.f, fused = 0.f, two = 0.f, matrix = 0.f, best = 0.f, generic = 0.f;
   auto time_z = [&] {
     if (f.hasRuns && fixedZ) {
       zr = time_launches([&] { z(1); }, ev.e0, ev.e1);
       ze = time_launches([&] { z(0); }, ev.e0, ev.e1);
       c.zRuns = zr <= ze ? 1 : 0;
-    } else if (fromValues > 0) {
+    } else if (fromValues > 0 || tryGeneric) {
       zr = ze = time_launches([&] { z(f.hasRuns); }, ev.e0, ev.e1);
     } else {
       z(f.hasRuns);
@@ -626,7 +681,6 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   };
   auto time_xy = [&] {
     const float zTime = fromValues > 0 ? std::min(zr, ze) : 0.f;
-    float best = 0.f;
     auto candidate = [&](bool serves, int plane, float* ms, auto&& run) {
       if (!serves) return;
       *ms = time_launches(run, ev.e0, ev.e1) + (plane == 3 ? 0.f : zTime);
@@ -646,14 +700,19 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
     time_z();
     time_xy();
   }
+  if (tryGeneric) {
+    generic = time_launches(
+        [&] { launch_generic(forward, f.in, f.out, f.useScale != 0, nullptr); }, ev.e0, ev.e1);
+    if (generic < best + (fromValues > 0 ? 0.f : std::min(zr, ze))) c.plane = kGenericKernels;
+  }
   tune_record(key, c);
   if (tune_log_enabled()) {
     std::fprintf(stderr, "spfft_amd tune: %s N=%d Nz=%d %s %s, single transform, %d columns: z "
-                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f, matrix %.4f ms -> "
-                 "plane=%d zruns=%d\n", sizeof(T) == 8 ? "double" : "float", map_->dimX,
+                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f, matrix %.4f, generic (all "
+                 "stages) %.4f ms -> plane=%d zruns=%d\n", sizeof(T) == 8 ? "double" : "float", map_->dimX,
                  map_->dimZ, map_->type == SPFFT_TRANS_R2C ? "R2C" : "C2C",
-                 forward ? "forward" : "backward", numCols_, zr, ze, fused, two, matrix, c.plane,
-                 c.zRuns);
+                 forward ? "forward" : "backward", numCols_, zr, ze, fused, two, matrix, generic,
+                 c.plane, c.zRuns);
   }
   return c;
 }
@@ -788,16 +847,18 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent, Famil
   hipEvent_t* ready = &ioEvents_[0];
   // of the FFT kernels, lengths that are not fixed have the generic ones only
   const bool fast = fast_ && (families == Families::kAll || tab_->fixedLengths);
-  if (!fast && !tab_->generic) throw InternalError();
-
+  const bool inPlace = overlap(inGPU, valueBytes, outGPU, space_domain_size() * sizeof(T));
+  FastArgs<T> f;
+  TuneChoice choice;
+  choice.plane = kGenericKernels;
   if (fast) {
-    FastArgs<T> f = fast_args();
+    f = fast_args();
     f.in = inGPU;
     f.out = outGPU;
-    const bool inPlace =
-        overlap(inGPU, valueBytes, outGPU, space_domain_size() * sizeof(T));
-    const TuneChoice choice = single_choice(
-        false, f, stream, inKind != MemKind::Device || hostOut || inPlace, families);
+    choice = single_choice(false, f, stream, inKind != MemKind::Device || hostOut || inPlace,
+                           families);
+  }
+  if (choice.plane != kGenericKernels) {
     // Values that lie in the field are all read before its first plane is written.
     const int fromValues = choice.plane == 3 && !inPlace ? from_values(false) : 0;
     if (fromValues == 0) {
@@ -819,23 +880,7 @@ void ExecutionGPU<T>::backward(const T* input, T* output, bool concurrent, Famil
       if (hostOut) check_hip(hipEventRecord(ready[c], stream));
     }
   } else {
-    StageArgs<T> a = base_args();
-    a.in = inGPU;
-    a.out = outGPU;
-    if (a.nst > 0) {
-      a.fft = fftZ_;
-      a.tw = tab_->twZ.data();
-      a.batch = zBatch_;
-      launch_z_backward<T>(a, stream);
-      a.fft = fftY_;
-      a.tw = tab_->twY.data();
-      a.batch = yBatch_;
-      launch_y_backward<T>(a, stream);
-    }
-    a.fft = fftX_;
-    a.tw = tab_->twX.data();
-    a.batch = xBatch_;
-    launch_x_backward<T>(a, stream);
+    launch_generic(false, inGPU, outGPU, false, stream);
     if (hostOut) {
       for (int c = 0; c < chunks; ++c) check_hip(hipEventRecord(ready[c], stream));
     }
@@ -884,14 +929,19 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
     if (copy != stream) check_hip(hipStreamWaitEvent(stream, done[c % kIoMaxChunks], 0));
   };
 
+  const bool useScale = scaling == SPFFT_FULL_SCALING;
+  FastArgs<T> f;
+  TuneChoice choice;
+  choice.plane = kGenericKernels;
   if (fast_) {
-    FastArgs<T> f = fast_args();
+    f = fast_args();
     f.in = inGPU;
     f.out = outGPU;
-    f.useScale = scaling == SPFFT_FULL_SCALING ? 1 : 0;
-    const TuneChoice choice =
-        single_choice(true, f, stream, hostIn || outKind != MemKind::Device ||
-                                           overlap(inGPU, spaceBytes, outGPU, valueBytes));
+    f.useScale = useScale ? 1 : 0;
+    choice = single_choice(true, f, stream, hostIn || outKind != MemKind::Device ||
+                                                overlap(inGPU, spaceBytes, outGPU, valueBytes));
+  }
+  if (choice.plane != kGenericKernels) {
     // host input: each chunk of planes is transformed as soon as it arrives
     for (int c = 0; c < chunks; ++c) {
       if (hostIn) upload_chunk(c);
@@ -918,24 +968,7 @@ void ExecutionGPU<T>::forward(const T* input, T* output, SpfftScalingType scalin
     // the ring is free again when the call returns (a later call refills it)
     check_hip(hipEventSynchronize(done[(chunks - 1) % kIoMaxChunks]));
   }
-  if (!fast_) {
-    StageArgs<T> a = base_args();
-    a.in = inGPU;
-    a.out = outGPU;
-    a.useScale = scaling == SPFFT_FULL_SCALING ? 1 : 0;
-    a.fft = fftX_;
-    a.tw = tab_->twX.data();
-    a.batch = xBatch_;
-    launch_x_forward<T>(a, stream);
-    a.fft = fftY_;
-    a.tw = tab_->twY.data();
-    a.batch = yBatch_;
-    launch_y_forward<T>(a, stream);
-    a.fft = fftZ_;
-    a.tw = tab_->twZ.data();
-    a.batch = zBatch_;
-    launch_z_forward<T>(a, stream);
-  }
+  if (choice.plane == kGenericKernels) launch_generic(true, inGPU, outGPU, useScale, stream);
   if (outKind != MemKind::Device) {
     hipEvent_t* ready = &ioEvents_[0];
     check_hip(hipEventRecord(ready[0], stream));
@@ -984,6 +1017,7 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
   shape->maxNcol = 0;
   shape->runs = true;
   shape->classSplit = shape->split = shape->matrix = shape->fixedLengths = true;
+  shape->tryGeneric = true;
   shape->fromValues = true;
   shape->maxNst = shape->kx = shape->ky = shape->kz = 0;
   for (size_t t = 0; t < n; ++t) {
@@ -992,6 +1026,7 @@ bool ExecutionGPU<T>::batch_qualifies(ExecutionGPU<T>* const* ex, size_t n, cons
     shape->split = shape->split && ex[t]->split_;
     shape->matrix = shape->matrix && ex[t]->matrix_;
     shape->fixedLengths = shape->fixedLengths && tab.fixedLengths;
+    shape->tryGeneric = shape->tryGeneric && tab.tryGeneric;
     shape->fromValues = shape->fromValues && tab.fromValues;
     shape->maxNst = std::max(shape->maxNst, ex[t]->map_->num_sticks());
     shape->kx = std::max(shape->kx, tab.kx);
@@ -1112,7 +1147,8 @@ void ExecutionGPU<T>::launch_batch(bool forward, const BatchShape& shape, int n,
 
 template <typename T>
 TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, int n, bool planeOk,
-                                       const FastArgs<T>* dArgs, const int2* dMap) {
+                                       const FastArgs<T>* dArgs, const int2* dMap,
+                                       const std::function<void()>& generic) {
   TuneChoice c;
   TuneEvents ev;
   auto z = [&](bool runs) {
@@ -1153,10 +1189,12 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
     zr = time_launches([&] { z(true); }, ev.e0, ev.e1);
     ze = time_launches([&] { z(false); }, ev.e0, ev.e1);
     c.zRuns = zr <= ze ? 1 : 0;
+  } else if (shape.tryGeneric) {
+    zr = ze = time_launches([&] { z(false); }, ev.e0, ev.e1);
   } else if (!forward) {
     z(false);
   }
-  float split = 0.f, plane0 = 0.f, plane1 = 0.f, two = 0.f, matrix = 0.f;
+  float split = 0.f, plane0 = 0.f, plane1 = 0.f, two = 0.f, matrix = 0.f, all = 0.f;
   float best = 1e30f;
   const size_t values = static_cast<size_t>(shape.dimX) * shape.dimY * shape.dimZ * n;
   const bool large = values * (shape.r2c ? 1 : 2) * sizeof(T) >= kStreamBatch;
@@ -1204,14 +1242,19 @@ TuneChoice ExecutionGPU<T>::tune_batch(bool forward, const BatchShape& shape, in
       }
     }
   }
+  if (shape.tryGeneric) {
+    all = time_launches(generic, ev.e0, ev.e1);
+    if (all < best + std::min(zr, ze)) c.plane = kGenericKernels;
+  }
   if (tune_log_enabled()) {
     std::fprintf(stderr,
                  "spfft_amd tune: %s N=%d Nz=%d %s %s, %d transforms, %d columns: z runs %.3f / "
                  "entries %.3f ms; class-split %.3f, split stage %.3f, whole-plane %.3f, one per "
-                 "CU %.3f, matrix %.3f ms -> plane=%d slots=%d zruns=%d\n",
+                 "CU %.3f, matrix %.3f, generic (all stages) %.3f ms -> plane=%d slots=%d "
+                 "zruns=%d\n",
                  sizeof(T) == 8 ? "double" : "float", shape.dimX, shape.dimZ,
                  shape.r2c ? "R2C" : "C2C", forward ? "forward" : "backward", n, shape.maxNcol,
-                 zr, ze, split, two, plane0, plane1, matrix, c.plane, c.slots, c.zRuns);
+                 zr, ze, split, two, plane0, plane1, matrix, all, c.plane, c.slots, c.zRuns);
   }
   return c;
 }
@@ -1299,11 +1342,18 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
 
   // kernel choices: forced plane family, recorded (this process or the cache
   // file), or timed now on this batch's buffers
+  shape.tryGeneric = shape.tryGeneric && !fft;
+  auto generic = [&] {
+    for (size_t t = 0; t < n; ++t) {
+      ex[t]->launch_generic(forward, din[t], dout[t], forward && scaling[t] == SPFFT_FULL_SCALING,
+                            nullptr);
+    }
+  };
   TuneChoice choice;
   const int forced = plane_kernels_forced();
   if (forced >= 0) {
     choice.plane = forced;
-  } else if (!shape.split && !(fixed_length(shape.dimZ) && shape.runs)) {
+  } else if (!shape.split && !(fixed_length(shape.dimZ) && shape.runs) && !shape.tryGeneric) {
     choice.plane = 3;  // nothing to choose
   } else {
     const TuneKey tkey = make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
@@ -1311,7 +1361,7 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
                                        shape.maxNcol, shape.maxNst, nt);
     // (timing would overwrite inputs that share memory with outputs)
     if (!tune_lookup(tkey, &choice) && !plan.inPlace) {
-      choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap);
+      choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap, generic);
       tune_record(tkey, choice);
     }
   }
@@ -1320,9 +1370,14 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
     choice.slots = 0;
   }
   if (choice.plane != 1) {
-    choice.plane = served_plane(choice.plane, shape.classSplit, shape.split, shape.matrix);
+    choice.plane = served_plane(choice.plane, shape.classSplit, shape.split, shape.matrix,
+                                shape.tryGeneric);
   }
-  launch_batch(forward, shape, nt, choice, dArgs, dMap, nullptr);
+  if (choice.plane == kGenericKernels) {
+    generic();
+  } else {
+    launch_batch(forward, shape, nt, choice, dArgs, dMap, nullptr);
+  }
   return true;
 }
 

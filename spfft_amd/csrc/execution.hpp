@@ -7,6 +7,7 @@
 
 #include <array>
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <vector>
 
@@ -35,6 +36,7 @@ struct TransformTables {
   bool allowFast = true;  // built with the fixed-length path allowed
   bool fast = false;      // fixed-length or matrix kernels serve this set
   bool generic = false;   // the generic kernels' tables are here
+  bool tryGeneric = false;  // the generic kernels may be faster: timed with the others
   bool split = false;     // the split plane stage does (fixed Nx and Ny)
   bool matrix = false;    // the matrix plane kernels do
   bool classSplit = false;    // the class-split plane kernels do (nx = ny, LDS fits)
@@ -97,6 +99,7 @@ public:
     bool classSplit = false;  // class-split plane kernels serve every transform
     bool split = false, matrix = false;  // the split stage, the matrix kernels do
     bool fixedLengths = false;           // all lengths are fixed ones
+    bool tryGeneric = false;             // the generic kernels are timed with the others
     bool fromValues = false;             // backward matrix kernels without a z kernel
     int maxNst = 0;                      // most sticks
     int kx = 0, ky = 0, kz = 0;          // largest centred indices
@@ -127,9 +130,10 @@ public:
                            const FastArgs<T>* dArgs, const int2* dMap, hipStream_t stream);
   // Times the candidate kernels on the batch's own buffers and returns the
   // fastest choice (the launches are idempotent; the call's real chain
-  // follows).
+  // follows). generic: enqueues the batch on the generic kernels.
   static TuneChoice tune_batch(bool forward, const BatchShape& shape, int n, bool planeOk,
-                               const FastArgs<T>* dArgs, const int2* dMap);
+                               const FastArgs<T>* dArgs, const int2* dMap,
+                               const std::function<void()>& generic);
 
   // run_batch for callers that cannot allocate (n >= 1 transforms). The
   // argument table and the z block map are written to `scratch`
@@ -177,6 +181,8 @@ private:
                 const hipEvent_t* ready, int readyCount, hipStream_t compute, hipStream_t copy);
   StageArgs<T> base_args() const;
   FastArgs<T> fast_args() const;
+  // The generic stage kernels (their tables are there), on device pointers.
+  void launch_generic(bool forward, const T* in, T* out, bool useScale, hipStream_t stream);
   // nz when the backward matrix kernels take the values themselves, else 0
   int from_values(bool forward) const {
     return !forward && tab_->fromValues ? map_->dimZ : 0;

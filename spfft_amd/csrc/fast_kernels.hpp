@@ -114,7 +114,8 @@ constexpr int fast_classes(int n) {
 // up to it, with or without fixed-length kernels. FP64 pairs at lengths without
 // fixed-length kernels, generic against matrix kernels: 143^3 136 / 101 us, 187^3
 // 842 / 205, 254^3 10317 / 796, 306^3 3833 / 1497, 343^3 1661 / 2765, 405^3 3462 /
-// 5019: past 306 the 7-smooth lengths run faster on the generic FFT.
+// 5019: the matrix kernels' work follows the square of a length. Of the smooth lengths
+// from 245 to 315 either may be faster: the tuner times both (execution.cpp).
 constexpr int kDftMaxLength = 320;
 
 // Geometry of the z kernels' LDS tile: sticks per workgroup, padded line
