@@ -629,7 +629,9 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   if (!split_ && !(fixedZ && f.hasRuns) && !tryGeneric) return c;
   const TuneKey key = make_tune_key(grid_->device_id(), static_cast<int>(sizeof(T)), map_->dimX,
                                     map_->dimY, map_->dimZ, map_->type == SPFFT_TRANS_R2C,
-                                    forward, fft, numCols_, map_->num_sticks(), 1);
+                                    forward, fft, f.hasRuns != 0,
+                                    mayMatrix && from_values(forward) > 0, numCols_,
+                                    map_->num_sticks(), 1);
   TuneChoice known;
   if (tune_lookup(key, &known)) {
     c.zRuns = known.zRuns && f.hasRuns;
@@ -1358,7 +1360,8 @@ bool ExecutionGPU<T>::run_batch(const std::vector<ExecutionGPU<T>*>& ex,
   } else {
     const TuneKey tkey = make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
                                        shape.dimY, shape.dimZ, shape.r2c, forward, fft,
-                                       shape.maxNcol, shape.maxNst, nt);
+                                       shape.runs, !forward && shape.fromValues, shape.maxNcol,
+                                       shape.maxNst, nt);
     // (timing would overwrite inputs that share memory with outputs)
     if (!tune_lookup(tkey, &choice) && !plan.inPlace) {
       choice = tune_batch(forward, shape, nt, planeOk, dArgs, dMap, generic);
@@ -1418,7 +1421,8 @@ void ExecutionGPU<T>::run_batch_noalloc(ExecutionGPU<T>* const* ex, size_t n, co
   } else {
     (void)tune_recorded(make_tune_key(shape.device, static_cast<int>(sizeof(T)), shape.dimX,
                                       shape.dimY, shape.dimZ, shape.r2c, forward, false,
-                                      shape.maxNcol, shape.maxNst, static_cast<int>(n)),
+                                      shape.runs, !forward && shape.fromValues, shape.maxNcol,
+                                      shape.maxNst, static_cast<int>(n)),
                         &choice);
   }
   if (choice.plane == 1 && !plane_candidate(ex, n, din, dout, forward, shape)) {

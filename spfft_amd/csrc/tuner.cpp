@@ -17,7 +17,7 @@ namespace spfft {
 
 namespace {
 
-using NumericKey = std::array<int, 11>;
+using NumericKey = std::array<int, 13>;
 
 struct TuneState {
   std::mutex mutex;
@@ -31,7 +31,8 @@ struct TuneState {
 
 NumericKey numeric(const TuneKey& k) {
   return {k.device,  k.valueBytes, k.n,          k.ny,          k.nz,         k.r2c,
-          k.forward, k.fft,        k.ncolBucket, k.stickBucket, k.countBucket};
+          k.forward, k.fft,        k.runs,       k.fromValues,  k.ncolBucket, k.stickBucket,
+          k.countBucket};
 }
 
 TuneState& state() {
@@ -53,7 +54,7 @@ std::string cache_path() {
   } else {
     return std::string();
   }
-  return base + "/spfft_amd/tune-v2.txt";
+  return base + "/spfft_amd/tune-v3.txt";
 }
 
 // mkdir -p of the directory part of `path`
@@ -94,8 +95,8 @@ void save_locked(const TuneState& s) {
   const std::string tmp = s.path + ".tmp" + std::to_string(static_cast<long>(getpid()));
   FILE* f = std::fopen(tmp.c_str(), "w");
   if (!f) return;
-  std::fprintf(f, "# spfft_amd kernel choices: <arch:CUs:bytes:N[xNy]:Nz:type:direction:"
-                  "columns:sticks:transforms> plane= slots= zruns=\n");
+  std::fprintf(f, "# spfft_amd kernel choices: <arch:CUs:bytes:N[xNy]:Nz:type:direction[:fft]:"
+                  "addressing[:values]:columns:sticks:transforms> plane= slots= zruns=\n");
   for (const auto& kv : s.choices) {
     std::fprintf(f, "%s plane=%d slots=%d zruns=%d\n", kv.first.c_str(), kv.second.plane,
                  kv.second.slots, kv.second.zRuns);
@@ -120,7 +121,7 @@ int round_quarter(int v) {
 }  // namespace
 
 TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2c, bool forward,
-                      bool fft, int maxNcol, int maxNst, int count) {
+                      bool fft, bool runs, bool fromValues, int maxNcol, int maxNst, int count) {
   TuneKey k;
   k.device = device;
   k.valueBytes = valueBytes;
@@ -130,6 +131,8 @@ TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2
   k.r2c = r2c ? 1 : 0;
   k.forward = forward ? 1 : 0;
   k.fft = fft ? 1 : 0;
+  k.runs = runs ? 1 : 0;
+  k.fromValues = fromValues ? 1 : 0;
   k.ncolBucket = (maxNcol + 15) / 16 * 16;
   k.stickBucket = round_quarter(maxNst);
   k.countBucket = round_pow2(count < 1 ? 1 : count);
@@ -162,7 +165,8 @@ std::string tune_key_text(const TuneKey& k) {
   o << arch << ":f" << 8 * k.valueBytes << ":N" << k.n;
   if (k.ny != k.n) o << "x" << k.ny;
   o << ":Z" << k.nz << ":"
-    << (k.r2c ? "r2c" : "c2c") << ":" << (k.forward ? "fwd" : "bwd") << (k.fft ? ":fft" : "") << ":col" << k.ncolBucket
+    << (k.r2c ? "r2c" : "c2c") << ":" << (k.forward ? "fwd" : "bwd") << (k.fft ? ":fft" : "")
+    << (k.runs ? ":runs" : ":entries") << (k.fromValues ? ":values" : "") << ":col" << k.ncolBucket
     << ":st" << k.stickBucket << ":x" << k.countBucket;
   return o.str();
 }

@@ -3,7 +3,9 @@
 // per-shape cache file, so later processes start from the measured choices.
 //
 // Key: device architecture and CU count, value bytes, Nx, Ny, Nz, C2C or R2C,
-// direction, whether the matrix kernels may run, widest column count (rounded up to 16), most sticks (rounded up to
+// direction, whether the matrix kernels may run, whether the sticks are runs and the
+// backward matrix kernels take the values themselves (both decide what is timed),
+// widest column count (rounded up to 16), most sticks (rounded up to
 // a quarter of an octave, since the work of a plane follows them) and transform
 // count (rounded up to a power of two; 1 for single transforms).
 // Choices: the plane-kernel family of batches (class-split kernels with R
@@ -15,8 +17,8 @@
 // value, or the per-value entry table).
 //
 // Cache file: SPFFT_AMD_TUNE_CACHE names it ("off" or empty: no file);
-// unset, $XDG_CACHE_HOME/spfft_amd/tune-v2.txt or ~/.cache/spfft_amd/
-// tune-v2.txt. One decision per line; unreadable lines are ignored; the file
+// unset, $XDG_CACHE_HOME/spfft_amd/tune-v3.txt or ~/.cache/spfft_amd/
+// tune-v3.txt. One decision per line; unreadable lines are ignored; the file
 // is replaced atomically (write, then rename) when a decision is added.
 #pragma once
 
@@ -29,7 +31,9 @@ struct TuneKey {
   int valueBytes = 0;
   int n = 0, ny = 0, nz = 0;
   int r2c = 0, forward = 0;
-  int fft = 0;  // without the matrix kernels
+  int fft = 0;         // without the matrix kernels
+  int runs = 0;        // the sticks are runs
+  int fromValues = 0;  // the backward matrix kernels need no z kernel
   int ncolBucket = 0, stickBucket = 0, countBucket = 0;
 };
 
@@ -42,7 +46,7 @@ struct TuneChoice {
 };
 
 TuneKey make_tune_key(int device, int valueBytes, int n, int ny, int nz, bool r2c, bool forward,
-                      bool fft, int maxNcol, int maxNst, int count);
+                      bool fft, bool runs, bool fromValues, int maxNcol, int maxNst, int count);
 // The recorded choice for `key` (from this process or the cache file).
 bool tune_lookup(const TuneKey& key, TuneChoice* choice);
 // Records a timed choice and rewrites the cache file.
