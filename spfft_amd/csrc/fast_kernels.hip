@@ -51,6 +51,7 @@ struct SplitCall {
   bool rc = false;                    // batches (single transforms: FastArgs::r2c)
   const FastArgs<T>* args = nullptr;  // the transform, or the batch's table
   int ntrans = 0, ny = 0, nz = 0, maxNcol = 0;  // batches
+  bool full = false;                  // batches: past kFullRegions
   hipStream_t stream = nullptr;
 };
 bool z_group0(int n, const ZCall<double>& c);
@@ -1503,7 +1504,9 @@ constexpr int split_waves() {
   return nw;
 }
 
-template <typename T, int N>
+// HALVES: with halved regions where they pay (see HALF_Y); batches of large fields have
+// kernels without them too (FULL_TOO).
+template <typename T, int N, bool HALVES = true>
 struct SplitShape {
   using L = FullLine<T, N>;
   static_assert(schedule_ok(N, L::E), "full line schedule");
@@ -1531,8 +1534,11 @@ struct SplitShape {
       kLdsMax / (static_cast<size_t>(tw_offset<T>(FULL)) * sizeof(Cx<T>) + N * sizeof(Tw<T>) +
                  N * sizeof(Cx<T>)) * NW);
   static constexpr bool HALF_Y =
-      sizeof(T) == 8 && N > 128 && dividing_schedule(N, L::E) && L::E % 2 == 0 && WAVES <= 12;
+      HALVES && sizeof(T) == 8 && N > 128 && dividing_schedule(N, L::E) && L::E % 2 == 0 && WAVES <= 12;
   static constexpr bool HALF_X = HALF_Y && N <= 256;
+  // Lengths whose batches past kFullRegions take full regions in both kernels: those
+  // without spare lanes, and with halved x kernels (192, 256; see kFullRegions).
+  static constexpr bool FULL_TOO = HALF_X && !L::SPARE;
   static constexpr int LBH = padded_len<float>(N);   // a line's halved region, in reals
   static constexpr int XH = (XL * LBH + 1) / 2;
   static constexpr int REGION_Y = !HALF_Y ? FULL : (XH > N / 2 * TP ? XH : N / 2 * TP);
@@ -1585,9 +1591,9 @@ __device__ __forceinline__ int stick_at(const int* table, int u, int y) {
   return table[(u * M + y % M) * R + y / M];
 }
 
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __device__ __forceinline__ void ysplit_backward_body(const FastArgs<T>& a, int bid) {
-  using S = SplitShape<T, N>;
+  using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
   constexpr int E = L::E, P = L::P;
   const int groups = S::col_groups(a.ncol);
@@ -1658,9 +1664,9 @@ __device__ __forceinline__ void ysplit_backward_body(const FastArgs<T>& a, int b
   }
 }
 
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int bid) {
-  using S = SplitShape<T, N>;
+  using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
   constexpr int E = L::E, P = L::P;
   const int ny = a.ny;  // rows of the plane (N is the row length)
@@ -1723,9 +1729,9 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   }
 }
 
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bid) {
-  using S = SplitShape<T, N>;
+  using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
   constexpr int E = L::E, P = L::P;
   const int ny = a.ny;  // rows of the plane (N is the row length)
@@ -1819,9 +1825,9 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool HALVES = true>
 __device__ __forceinline__ void ysplit_forward_body(const FastArgs<T>& a, int bid) {
-  using S = SplitShape<T, N>;
+  using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
   constexpr int E = L::E, P = L::P;
   const int groups = S::col_groups(a.ncol);
@@ -2041,29 +2047,29 @@ template <typename T, int N>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_ysplit_forward(FastArgs<T> a) {
   ysplit_forward_body<T, N>(a, blockIdx.x);
 }
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_ysplit_backward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  ysplit_backward_body<T, N, RC>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  ysplit_backward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_backward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_backward_body<T, N, RC>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_backward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_forward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_forward_body<T, N, RC>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_forward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
-template <typename T, int N>
+template <typename T, int N, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_ysplit_forward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  ysplit_forward_body<T, N>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  ysplit_forward_body<T, N, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
 
 template <typename T, int N>
@@ -2692,9 +2698,9 @@ int plane_xy_slots(bool forward, int n) {
 
 // ---- split plane stage launches
 
-template <typename T, int N, bool Y, typename Kernel, typename... Args>
+template <typename T, int N, bool Y, bool HALVES = true, typename Kernel, typename... Args>
 void split_launch(Kernel kernel, const char* name, int blocks, hipStream_t stream, Args... args) {
-  using S = SplitShape<T, N>;
+  using S = SplitShape<T, N, HALVES>;
   prepare_lds(kernel, S::lds(Y));
   prof::KernelSpan span(stream, name, true);
   hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(S::NT), S::lds(Y), stream, span.start(),
@@ -2730,33 +2736,49 @@ void xsplit_n(bool forward, const FastArgs<T>& a, hipStream_t stream) {
         "k_xsplit_backward", blocks, stream, a);
   }
 }
-template <typename T, int NY>
+template <typename T, int NY, bool HALVES>
 void ysplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans, int nz,
                     int maxNcol, hipStream_t stream) {
-  using S = SplitShape<T, NY>;
+  using S = SplitShape<T, NY, HALVES>;
   const int per = S::col_groups(maxNcol) * nz;
   if (forward) {
-    split_launch<T, NY, true>(k_ysplit_forward_batch<T, NY>, "k_ysplit_forward_batch", per * ntrans,
-                        stream, batch, per);
+    split_launch<T, NY, true, HALVES>(
+        k_ysplit_forward_batch<T, NY, HALVES>,
+        HALVES ? "k_ysplit_forward_batch" : "k_ysplit_forward_batch_full", per * ntrans, stream,
+        batch, per);
   } else {
-    split_launch<T, NY, true>(rc ? k_ysplit_backward_batch<T, NY, true>
-                           : k_ysplit_backward_batch<T, NY, false>,
-                        "k_ysplit_backward_batch", per * ntrans, stream, batch, per);
+    split_launch<T, NY, true, HALVES>(
+        rc ? k_ysplit_backward_batch<T, NY, true, HALVES>
+           : k_ysplit_backward_batch<T, NY, false, HALVES>,
+        HALVES ? "k_ysplit_backward_batch" : "k_ysplit_backward_batch_full", per * ntrans, stream,
+        batch, per);
   }
 }
-template <typename T, int NX>
+template <typename T, int NX, bool HALVES>
 void xsplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans, int ny, int nz,
                     hipStream_t stream) {
-  using S = SplitShape<T, NX>;
+  using S = SplitShape<T, NX, HALVES>;
   const int per = S::row_groups(ny, rc) * nz;
   if (forward) {
-    split_launch<T, NX, false>(rc ? k_xsplit_forward_batch<T, NX, true>
-                           : k_xsplit_forward_batch<T, NX, false>,
-                        "k_xsplit_forward_batch", per * ntrans, stream, batch, per);
+    split_launch<T, NX, false, HALVES>(
+        rc ? k_xsplit_forward_batch<T, NX, true, HALVES>
+           : k_xsplit_forward_batch<T, NX, false, HALVES>,
+        HALVES ? "k_xsplit_forward_batch" : "k_xsplit_forward_batch_full", per * ntrans, stream,
+        batch, per);
   } else {
-    split_launch<T, NX, false>(rc ? k_xsplit_backward_batch<T, NX, true>
-                           : k_xsplit_backward_batch<T, NX, false>,
-                        "k_xsplit_backward_batch", per * ntrans, stream, batch, per);
+    split_launch<T, NX, false, HALVES>(
+        rc ? k_xsplit_backward_batch<T, NX, true, HALVES>
+           : k_xsplit_backward_batch<T, NX, false, HALVES>,
+        HALVES ? "k_xsplit_backward_batch" : "k_xsplit_backward_batch_full", per * ntrans, stream,
+        batch, per);
+  }
+}
+template <typename T, int N, bool HALVES>
+void split_batch_call(const SplitCall<T>& c) {
+  if (c.y) {
+    ysplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.nz, c.maxNcol, c.stream);
+  } else {
+    xsplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.stream);
   }
 }
 
@@ -2780,10 +2802,11 @@ void split_call(const SplitCall<T>& c) {
     } else {
       xsplit_n<T, N>(c.forward, *c.args, c.stream);
     }
-  } else if (c.y) {
-    ysplit_batch_n<T, N>(c.forward, c.rc, c.args, c.ntrans, c.nz, c.maxNcol, c.stream);
   } else {
-    xsplit_batch_n<T, N>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.stream);
+    if constexpr (SplitShape<T, N>::FULL_TOO) {
+      if (c.full) return split_batch_call<T, N, false>(c);
+    }
+    split_batch_call<T, N, true>(c);
   }
 }
 
@@ -2811,6 +2834,7 @@ void launch_split_xy(bool forward, int nx, int ny, const FastArgs<T>& a, hipStre
 template <typename T>
 void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArgs<T>* batch,
                            int ntrans, int nz, int maxNcol, hipStream_t stream) {
+  const size_t bytes = sizeof(T) * (r2c ? 1 : 2) * nx * ny * nz * ntrans;
   for (int k = 0; k < 2; ++k) {
     SplitCall<T> c;
     c.y = (k == 0) != forward;
@@ -2822,6 +2846,7 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
     c.ny = ny;
     c.nz = nz;
     c.maxNcol = maxNcol;
+    c.full = bytes >= kFullRegions;
     c.stream = stream;
     split_dispatch(c.y ? ny : nx, c);
   }

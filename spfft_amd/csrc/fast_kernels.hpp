@@ -103,6 +103,15 @@ constexpr size_t kStreamBatch = size_t{144} << 20;
 // streaming loads, which keep it out of the column buffer's way (256^3 FP64 pair 266
 // / 255 us plain / streaming; within the cache, 224^3 FP64, 237 / 240).
 constexpr size_t kLastLevelCache = size_t{256} << 20;
+// Batches of this much space domain run the split stage with full LDS regions at 192 and
+// 256 (SplitShape::FULL_TOO; FP64): they are bound by HBM, where more waves per CU only
+// add to the streams in flight. Pairs, us, halved / full, radius 0.3125 N: 5 x 192^3 (540
+// MiB) 755 / 749, 6 x 897 / 880, 8 x 1184 / 1157, 2 x 256^3 (512 MiB) 695 / 679, 4 x
+// 1372 / 1349, 4 x 256^3 R2C (512 MiB) 713 / 705; below, 3 x 192^3 418 / 436, 4 x 192^3
+// (432 MiB) 602 / 606. The lengths with spare lanes keep the halves: 4 x 216^3 (615 MiB)
+// 1021 / 1130, 4 x 200^3 780 / 863; so do longer ones, whose x kernels have full regions
+// anyway: 2 x 320^3 1363 / 1390.
+constexpr size_t kFullRegions = size_t{512} << 20;
 
 // Residue classes per plane used by the xy kernels of length n.
 // (A divisor of n: the stick index table is class-interleaved with it.)
