@@ -172,6 +172,8 @@ std::string tune_key_text(const TuneKey& k) {
 }
 
 bool tune_lookup(const TuneKey& key, TuneChoice* choice) {
+  // every call but a shape's first in the process: no text to build
+  if (tune_recorded(key, choice)) return true;
   const std::string text = tune_key_text(key);
   TuneState& s = state();
   std::lock_guard<std::mutex> lock(s.mutex);
