@@ -622,8 +622,9 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   c.plane = served_plane(forced, classSplit_, split_, mayMatrix);
   if (forced >= 0) return c;
   const bool tryGeneric = tab_->tryGeneric && !fft;
-  // batched fallbacks on the transform's own stream keep the defaults
-  if (stream != nullptr) return c;
+  // batched fallbacks on the transform's own stream keep the defaults (between the
+  // generic and the matrix kernels: a recorded choice)
+  if (stream != nullptr && !tryGeneric) return c;
   const bool fixedZ = fixed_length(map_->dimZ);
   // nothing to choose
   if (!split_ && !(fixedZ && f.hasRuns) && !tryGeneric) return c;
@@ -641,11 +642,12 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   // Timing would overwrite host data staged in the work buffer (by the split
   // stage's column buffer) and an input that shares memory with the output: no
   // timing on such a call (defaults).
-  if (keepInput) return c;
-  // Every launch below is idempotent, its input and output apart: backward z reads the values and writes
-  // the [z][stick] buffer, the plane stage reads that buffer and writes the
-  // output; forward the plane stage reads the input and writes the buffer,
-  // z reads it and writes the values. The call's real launches follow.
+  if (keepInput || stream != nullptr) return c;
+  // Every launch below is idempotent, its input and output apart: backward z
+  // reads the values and writes the [z][stick] buffer, the plane stage reads that
+  // buffer and writes the output; forward the plane stage reads the input and
+  // writes the buffer, z reads it and writes the values. The call's real launches
+  // follow.
   TuneEvents ev;
   FastArgs<T> a = f;
   a.zBegin = 0;

@@ -1,7 +1,7 @@
 """Sets with a long line that is not of a fixed length, all lengths without prime
 factors above 13: the first call times the generic kernels against the matrix kernels
 and keeps the faster (single transforms and batches), and either choice, once
-recorded, is the one that runs. Outputs are checked against the oracle each time.
+recorded, is the one that runs, also for one transform in a multi-transform call. Outputs are checked against the oracle each time.
 
 Each part runs in a fresh process, since the choices are per process. Tolerances: those
 of the generic kernels, 1e-12 (FP64) and 1e-5 (FP32)."""
@@ -29,10 +29,11 @@ from tests.test_gpu_parity import build
 from tests.test_gpu_split_lengths import kernels_run
 from tests.workloads import complex_values
 
-for dims, r2c, precision, count in (((245, 24, 18), False, "double", 1),
-                                    ((20, 18, 250), True, "float", 1),
-                                    ((16, 308, 24), True, "double", 3),
-                                    ((35, 176, 24), False, "float", 2)):
+for dims, r2c, precision, count, multi in (((245, 24, 18), False, "double", 1, False),
+                                           ((20, 18, 250), True, "float", 1, False),
+                                           ((16, 308, 24), True, "double", 3, True),
+                                           ((35, 176, 24), False, "float", 2, True),
+                                           ((245, 24, 18), False, "double", 1, True)):
     print("case", dims, count, flush=True)
     t = ellipsoid(dims, 0.4, r2c)
     o = orc.OraclePlan(r2c, dims, t)
@@ -45,7 +46,7 @@ for dims, r2c, precision, count in (((245, 24, 18), False, "double", 1),
     outs = [torch.empty(2 * len(t), dtype=dt, device="cuda") for _ in vals]
     trs = [build(dims, t, r2c, precision) for _ in vals]
     def run():
-        if count == 1:
+        if not multi:
             trs[0].backward(ins[0], spaces[0])
             trs[0].forward(spaces[0], outs[0], sp.SPFFT_FULL_SCALING)
         else:
@@ -87,7 +88,7 @@ def test_either_choice_runs(tmp_path):
         cache.write_text(re.sub(r"plane=\d", f"plane={plane}", text))
         log, ran = run_child(tmp_path, cache)
         assert "spfft_amd tune:" not in log, log
-        assert len(ran) == 4
+        assert len(ran) == 5
         for names in ran:
             names = " ".join(names) + " "
             assert stage in names and other not in names, (plane, names)
