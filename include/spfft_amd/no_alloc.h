@@ -19,11 +19,11 @@
  *    fixed-length kernels (Nx = Ny in {32, 64, 96, 128, 192}), with non-empty
  *    index sets;
  *  - every input and output pointer in device memory;
- *  - the tables fit in SPFFT_AMD_NOALLOC_SCRATCH_BYTES (1 MiB): 224 bytes per
+ *  - the tables fit in SPFFT_AMD_NOALLOC_SCRATCH_BYTES (1 MiB): 248 bytes per
  *    transform (the total padded to 256) plus 8 bytes per block of sticks,
  *    a block holding 8 sticks at Nz = 128, 16 at Nz = 64 and 192, 32 at
- *    Nz = 32 and 96. Examples: up to 199 transforms of 128^3 with a radius-40
- *    sphere (5,025 sticks), up to 178 of 192^3 with radius 60 (11,289 sticks).
+ *    Nz = 32 and 96. Examples: up to 198 transforms of 128^3 with a radius-40
+ *    sphere (5,025 sticks), up to 177 of 192^3 with radius 60 (11,289 sticks).
  * A null handle in the array is SPFFT_INVALID_PARAMETER_ERROR, as in the
  * multi_transform functions.
  *

@@ -270,7 +270,8 @@ def _energy_gradient(transforms, psi, own, potential, grad_energy):
     field = psi if own else torch.empty_like(psi)
     sp._check(sp.lib.spfft_amd_energy_field(
         psi.device.index, potential.element_size(), psi.data_ptr(), potential.data_ptr(), scale,
-        potential.numel(), psi.shape[0], field.data_ptr(), torch.cuda.current_stream(psi.device).cuda_stream), "energy_field")
+        potential.numel(), psi.shape[0], field.data_ptr(),
+        torch.cuda.current_stream(psi.device).cuda_stream), "energy_field")
     g = _batch_adjoint(transforms, n, field)
     return g if scale is not None else grad_energy.to(potential.dtype) * g
 

@@ -9,7 +9,7 @@
 
 namespace spfft {
 
-// Device array per GPU: one argument table (224 bytes per FP64 transform,
+// Device array per GPU: one argument table (248 bytes per FP64 transform,
 // padded to 256 bytes in total) and one z block map (8 bytes per block of
 // sticks).
 constexpr size_t kNoAllocScratchBytes = size_t(1) << 20;
