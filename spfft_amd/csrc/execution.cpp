@@ -562,7 +562,7 @@ FastArgs<T> ExecutionGPU<T>::fast_args() const {
   a.zInfo = tab_->zInfo.data();
   a.hasRuns = tab_->zInfo.data() != nullptr ? 1 : 0;
   const size_t bytes = space_domain_size() * sizeof(T);
-  a.streamOut = bytes >= kStreamField ? 1 : 0;
+  a.streamOut = bytes >= kStreamField ? 2 : (bytes >= kStreamHalved ? 1 : 0);
   a.pastCache = bytes >= kLastLevelCache ? 1 : 0;
   a.pitchT = pitchT_;
   a.resYM = tab_->resYM.data();
@@ -1100,7 +1100,7 @@ void ExecutionGPU<T>::fill_batch_tables(ExecutionGPU<T>* const* ex, size_t n, co
     f.in = din[t];
     f.out = dout[t];
     f.useScale = forward && scaling[t] == SPFFT_FULL_SCALING ? 1 : 0;
-    f.streamOut = bytes >= kStreamBatch ? 1 : 0;
+    f.streamOut = bytes >= kStreamBatch ? 2 : 0;
     f.pastCache = bytes >= kLastLevelCache ? 1 : 0;
     f.pitchA = ex[t]->classSplit_ ? fast_xy_pitch_a<T>(ex[0]->map_->dimX, f.ncol) : 0;
     if (zmap) {

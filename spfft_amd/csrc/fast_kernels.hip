@@ -52,6 +52,7 @@ struct SplitCall {
   const FastArgs<T>* args = nullptr;  // the transform, or the batch's table
   int ntrans = 0, ny = 0, nz = 0, maxNcol = 0;  // batches
   bool full = false;                  // batches: past kFullRegions
+  bool pastCache = false;             // batches: past kLastLevelCache
   hipStream_t stream = nullptr;
 };
 bool z_group0(int n, const ZCall<double>& c);
@@ -402,17 +403,15 @@ __device__ __forceinline__ void store_line(bool stream, V* p, F value) {
   }
 }
 
-// The same for the loads of a row (see kLastLevelCache).
-template <int E, int P, typename V, typename F>
-__device__ __forceinline__ void load_line(bool stream, const V* p, F take) {
-  if (stream) {
-    apart();
-#pragma unroll
-    for (int e = 0; e < E; ++e) take(e, load_stream(p + P * e));
-    apart();
+// A load of the space domain. Streaming ones (see kLastLevelCache) are a kernel of
+// their own: as a branch inside one kernel they cost the plain loads registers and
+// waits, 2 to 14 % of the forward call (416 x 416 x 64 R2C FP64 95 -> 111 us).
+template <bool STREAM, typename V>
+__device__ __forceinline__ V load(const V* p) {
+  if constexpr (STREAM) {
+    return load_stream(p);
   } else {
-#pragma unroll
-    for (int e = 0; e < E; ++e) take(e, p[P * e]);
+    return *p;
   }
 }
 
@@ -1151,11 +1150,11 @@ __device__ __forceinline__ void xy_backward_body(const FastArgs<T>& a, int bid) 
       if (RC) {
         // row b = row a + R rows
         T* rowB = a.out + row + static_cast<size_t>(R) * N;
-        store_line<LX::E, LX::P>(a.streamOut, a.out + row + q, [&](int e) { return v[e].re; });
-        store_line<LX::E, LX::P>(a.streamOut, rowB + q, [&](int e) { return v[e].im; });
+        store_line<LX::E, LX::P>(a.streamOut > 1, a.out + row + q, [&](int e) { return v[e].re; });
+        store_line<LX::E, LX::P>(a.streamOut > 1, rowB + q, [&](int e) { return v[e].im; });
       } else {
         Cx<T>* out = reinterpret_cast<Cx<T>*>(a.out) + row;
-        store_line<LX::E, LX::P>(a.streamOut, out + q, [&](int e) { return v[e]; });
+        store_line<LX::E, LX::P>(a.streamOut > 1, out + q, [&](int e) { return v[e]; });
       }
     }
   }
@@ -1717,19 +1716,20 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twX[t];
   __syncthreads();
   S::template fft<true, S::HALF_X>(v, region, wave, lane, twl);
+  const bool stream = a.streamOut > (S::HALF_X ? 0 : 1);
   if (y < ny) {
     const size_t row = (static_cast<size_t>(z) * ny + y) * N;
     if (RC) {
-      store_line<E, P>(a.streamOut, a.out + row + q, [&](int e) { return v[e].re; });
-      if (hasB) store_line<E, P>(a.streamOut, a.out + row + N + q, [&](int e) { return v[e].im; });
+      store_line<E, P>(stream, a.out + row + q, [&](int e) { return v[e].re; });
+      if (hasB) store_line<E, P>(stream, a.out + row + N + q, [&](int e) { return v[e].im; });
     } else {
       Cx<T>* out = reinterpret_cast<Cx<T>*>(a.out) + row;
-      store_line<E, P>(a.streamOut, out + q, [&](int e) { return v[e]; });
+      store_line<E, P>(stream, out + q, [&](int e) { return v[e]; });
     }
   }
 }
 
-template <typename T, int N, bool RC, bool HALVES = true>
+template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bid) {
   using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
@@ -1754,11 +1754,15 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   Cx<T> v[E];
   if (RC) {
     const size_t rowB = hasB ? row + N : row;
-    load_line<E, P>(a.pastCache, a.in + row + q, [&](int e, T x) { v[e].re = x; });
-    load_line<E, P>(a.pastCache, a.in + rowB + q, [&](int e, T x) { v[e].im = hasB ? x : T(0); });
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const T b = load<STREAM>(a.in + rowB + q + P * e);
+      v[e] = Cx<T>{load<STREAM>(a.in + row + q + P * e), hasB ? b : T(0)};
+    }
   } else {
     const Cx<T>* in = reinterpret_cast<const Cx<T>*>(a.in) + row;
-    load_line<E, P>(a.pastCache, in + q, [&](int e, Cx<T> x) { v[e] = x; });
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = load<STREAM>(in + q + P * e);
   }
   int uu[E];
 #pragma unroll
@@ -1770,9 +1774,10 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
     // Z = A + i B with A, B the spectra of the real rows a and b:
     // A[x] = (Z[x] + conj Z[N - x]) / 2, B[x] = -i (Z[x] - conj Z[N - x]) / 2.
     // The partner of x is held by lane (P - q) % P; it comes through the
-    // line's exchange region (wave-local; real, then imaginary parts in a
-    // halved one).
-    Cx<T> partner[E];
+    // line's exchange region (wave-local; of a halved one, real and imaginary
+    // parts in turn through registers).
+    Cx<T> partner[S::HALF_X ? E : 1];
+    const Cx<T>* whole = S::xregion(region, wave, lane);
     wave_sync();
     if constexpr (S::HALF_X) {
       T* lr = S::hregion(region, wave, lane);
@@ -1798,18 +1803,19 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
 #pragma unroll
       for (int e = 0; e < E; ++e) lr[phys<T>(q + P * e)] = v[e];
       wave_sync();
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int x = q + P * e;
-        partner[e] = lr[phys<T>(x == 0 ? 0 : N - x)];
-      }
     }
     if (y < ny) {
       Cx<T>* ya = a.ybuf + (static_cast<size_t>(z) * ny + y) * a.pitchY;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
+        const int x = q + P * e;
         if (uu[e] < a.ncol) {
-          const Cx<T> zp = partner[e];
+          Cx<T> zp;
+          if constexpr (S::HALF_X) {
+            zp = partner[e];
+          } else {
+            zp = whole[phys<T>(x == 0 ? 0 : N - x)];
+          }
           const T h = T(0.5);
           ya[uu[e]] = Cx<T>{h * (v[e].re + zp.re), h * (v[e].im - zp.im)};
           if (hasB) ya[a.pitchY + uu[e]] = Cx<T>{h * (v[e].im + zp.im), h * (zp.re - v[e].re)};
@@ -2039,9 +2045,9 @@ template <typename T, int N, bool RC>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_xsplit_backward(FastArgs<T> a) {
   xsplit_backward_body<T, N, RC>(a, blockIdx.x);
 }
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool STREAM>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_xsplit_forward(FastArgs<T> a) {
-  xsplit_forward_body<T, N, RC>(a, blockIdx.x);
+  xsplit_forward_body<T, N, RC, STREAM>(a, blockIdx.x);
 }
 template <typename T, int N>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_ysplit_forward(FastArgs<T> a) {
@@ -2059,11 +2065,11 @@ __global__ void __launch_bounds__((SplitShape<T, N>::NT))
   const int t = blockIdx.x / perTransform;
   xsplit_backward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
-template <typename T, int N, bool RC, bool HALVES = true>
+template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_forward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_forward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_forward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
 template <typename T, int N, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
@@ -2727,9 +2733,11 @@ void xsplit_n(bool forward, const FastArgs<T>& a, hipStream_t stream) {
   using S = SplitShape<T, NX>;
   const int blocks = S::row_groups(a.ny, a.r2c != 0) * (a.nz - a.zBegin);
   if (forward) {
-    split_launch<T, NX, false>(
-        a.r2c ? k_xsplit_forward<T, NX, true> : k_xsplit_forward<T, NX, false>,
-        "k_xsplit_forward", blocks, stream, a);
+    auto kernel = a.pastCache ? (a.r2c ? k_xsplit_forward<T, NX, true, true>
+                                       : k_xsplit_forward<T, NX, false, true>)
+                              : (a.r2c ? k_xsplit_forward<T, NX, true, false>
+                                       : k_xsplit_forward<T, NX, false, false>);
+    split_launch<T, NX, false>(kernel, "k_xsplit_forward", blocks, stream, a);
   } else {
     split_launch<T, NX, false>(
         a.r2c ? k_xsplit_backward<T, NX, true> : k_xsplit_backward<T, NX, false>,
@@ -2756,15 +2764,21 @@ void ysplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans,
 }
 template <typename T, int NX, bool HALVES>
 void xsplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans, int ny, int nz,
-                    hipStream_t stream) {
+                    bool pastCache, hipStream_t stream) {
   using S = SplitShape<T, NX, HALVES>;
   const int per = S::row_groups(ny, rc) * nz;
   if (forward) {
+    auto kernel = rc ? k_xsplit_forward_batch<T, NX, true, true, HALVES>
+                     : k_xsplit_forward_batch<T, NX, false, true, HALVES>;
+    if constexpr (HALVES) {  // full regions: past the cache
+      if (!pastCache) {
+        kernel = rc ? k_xsplit_forward_batch<T, NX, true, false, HALVES>
+                    : k_xsplit_forward_batch<T, NX, false, false, HALVES>;
+      }
+    }
     split_launch<T, NX, false, HALVES>(
-        rc ? k_xsplit_forward_batch<T, NX, true, HALVES>
-           : k_xsplit_forward_batch<T, NX, false, HALVES>,
-        HALVES ? "k_xsplit_forward_batch" : "k_xsplit_forward_batch_full", per * ntrans, stream,
-        batch, per);
+        kernel, HALVES ? "k_xsplit_forward_batch" : "k_xsplit_forward_batch_full", per * ntrans,
+        stream, batch, per);
   } else {
     split_launch<T, NX, false, HALVES>(
         rc ? k_xsplit_backward_batch<T, NX, true, HALVES>
@@ -2778,7 +2792,8 @@ void split_batch_call(const SplitCall<T>& c) {
   if (c.y) {
     ysplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.nz, c.maxNcol, c.stream);
   } else {
-    xsplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.stream);
+    xsplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.pastCache,
+                                 c.stream);
   }
 }
 
@@ -2847,6 +2862,7 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
     c.nz = nz;
     c.maxNcol = maxNcol;
     c.full = bytes >= kFullRegions;
+    c.pastCache = bytes >= kLastLevelCache;
     c.stream = stream;
     split_dispatch(c.y ? ny : nx, c);
   }
@@ -2905,6 +2921,7 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
 #define SPFFT_FAST_UNIT 0
 #endif
 #if SPFFT_FAST_UNIT == 0
+static_assert(kFullRegions >= kLastLevelCache, "full regions stream their loads");
 bool fixed_length(int n) { return square_length(n) || split_only_length(n); }
 SPFFT_INSTANTIATE_FAST_PLANE(double)
 #elif SPFFT_FAST_UNIT == 1

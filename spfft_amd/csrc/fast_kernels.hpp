@@ -65,7 +65,8 @@ struct FastArgs {
                                       // every stick's values are one run in user order
   int hasRuns = 0;                    // zInfo is valid (set on the host; kernels select the
                                       // stick-run path on this flag, never on the pointer)
-  int streamOut = 0;                  // backward: streaming stores of the space domain
+  int streamOut = 0;                  // backward, streaming stores of the space domain: 2, or 1
+                                      // by halved x kernels only (kStreamHalved)
   const int* xCol = nullptr;          // [NX]: column id of x, or ncol (a zero column)
   const int* resSticks = nullptr;     // sticks grouped by colX mod R
   const int* resBegin = nullptr;      // R + 1 offsets into resSticks
@@ -86,10 +87,13 @@ struct FastArgs {
 // it there for the next call to read; more, and the field only pushes out the stick
 // and column buffers that the launch's own kernels pass on, and its write-back falls
 // into the next launch. All times us, plain / streaming stores:
-//   one transform, from 96 MiB: pairs 256^3 FP64 300 / 256, 240^3 FP64 (211 MiB)
-//     289 / 276, 216^3 FP64 (154 MiB) 240 / 238, 256^3 FP32 (128 MiB) 157 / 159;
-//     backward alone 192^3 FP64 (108 MiB) 80 / 72, 256^3 FP32 92 / 70; below that
-//     (128^3 FP64, 32 MiB) 42.4 / 44.5 per pair;
+//   one transform, from 136 MiB: pairs (over three fields in turn) 256^3 FP64 306 / 283,
+//     240^3 FP64 (211 MiB) 328 / 307, 216^3 (154 MiB) 250 / 245, 210^3 (141 MiB) 243 / 238,
+//     208^3 (137 MiB) even; below, a pair's forward call finds the field in the cache:
+//     198^3 (118 MiB) 266 / 270, 360 x 360 x 64 (127 MiB) 241 / 244, 240^3 FP32 (105 MiB)
+//     168 / 170, 240^3 R2C 184 / 187, 192^3 class-split 278 / 290 (backward alone gains
+//     2 to 10 % from 96 MiB on). The x kernels with halved regions (192, 200) from 96 MiB:
+//     pairs 192^3 (108 MiB) 150.7 / 149.5, 200^3 even, backward alone 80 / 73, 97 / 90;
 //   batches, from 144 MiB: 3 x 192^3 FP64 (324 MiB) 399 / 356, 8 x 128^3 FP64
 //     (256 MiB) 240 / 228, 8 x 144^3 FP32 (182 MiB) 280 / 264, 8 x 128^3 R2C
 //     (128 MiB) 154 / 155, 60 x 64^3 R2C (120 MiB) 142 / 148.
@@ -97,7 +101,8 @@ struct FastArgs {
 // stream once the space domain is past the cache (12 x 120^3, 316 MiB, 365 / 342; 11 x
 // 100^3, 168 MiB, 192 / 218), 128 and 64 bytes for the other types, which stay plain
 // (12 x 120^3 R2C 226 / 251).
-constexpr size_t kStreamField = size_t{96} << 20;
+constexpr size_t kStreamField = size_t{136} << 20;
+constexpr size_t kStreamHalved = size_t{96} << 20;
 constexpr size_t kStreamBatch = size_t{144} << 20;
 // Forward: the split stage's x kernel reads a space domain past the cache with
 // streaming loads, which keep it out of the column buffer's way (256^3 FP64 pair 266
