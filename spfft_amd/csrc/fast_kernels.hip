@@ -51,8 +51,7 @@ struct SplitCall {
   bool rc = false;                    // batches (single transforms: FastArgs::r2c)
   const FastArgs<T>* args = nullptr;  // the transform, or the batch's table
   int ntrans = 0, ny = 0, nz = 0, maxNcol = 0;  // batches
-  bool full = false;                  // batches: past kFullRegions
-  bool pastCache = false;             // batches: past kLastLevelCache
+  size_t bytes = 0;                   // batches: their space domain
   hipStream_t stream = nullptr;
 };
 bool z_group0(int n, const ZCall<double>& c);
@@ -400,6 +399,15 @@ __device__ __forceinline__ void store_line(bool stream, V* p, F value) {
   } else {
 #pragma unroll
     for (int e = 0; e < E; ++e) p[P * e] = value(e);
+  }
+}
+
+template <bool STREAM, typename V>
+__device__ __forceinline__ void store(V* p, V v) {
+  if constexpr (STREAM) {
+    store_stream(p, v);
+  } else {
+    *p = v;
   }
 }
 
@@ -1538,6 +1546,10 @@ struct SplitShape {
   // Lengths whose batches past kFullRegions take full regions in both kernels: those
   // without spare lanes, and with halved x kernels (192, 256; see kFullRegions).
   static constexpr bool FULL_TOO = HALF_X && !L::SPARE;
+  // True when a backward call of one transform stores its rows past the cache.
+  __host__ __device__ static constexpr bool streams(int streamOut) {
+    return streamOut > (HALF_X ? 0 : 1);
+  }
   static constexpr int LBH = padded_len<float>(N);   // a line's halved region, in reals
   static constexpr int XH = (XL * LBH + 1) / 2;
   static constexpr int REGION_Y = !HALF_Y ? FULL : (XH > N / 2 * TP ? XH : N / 2 * TP);
@@ -1663,7 +1675,10 @@ __device__ __forceinline__ void ysplit_backward_body(const FastArgs<T>& a, int b
   }
 }
 
-template <typename T, int N, bool RC, bool HALVES = true>
+// STREAM: streaming stores of real rows, in kernels of their own (as a branch they cost
+// the plain ones 3 to 10 %: 132^3 FP32 12.7 -> 13.9 us, 180^3 16.0 -> 16.7); those of
+// complex rows, which a branch does not slow, go by FastArgs::streamOut.
+template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int bid) {
   using S = SplitShape<T, N, HALVES>;
   using L = typename S::L;
@@ -1716,15 +1731,18 @@ __device__ __forceinline__ void xsplit_backward_body(const FastArgs<T>& a, int b
   for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twX[t];
   __syncthreads();
   S::template fft<true, S::HALF_X>(v, region, wave, lane, twl);
-  const bool stream = a.streamOut > (S::HALF_X ? 0 : 1);
   if (y < ny) {
     const size_t row = (static_cast<size_t>(z) * ny + y) * N;
-    if (RC) {
-      store_line<E, P>(stream, a.out + row + q, [&](int e) { return v[e].re; });
-      if (hasB) store_line<E, P>(stream, a.out + row + N + q, [&](int e) { return v[e].im; });
+    if constexpr (RC) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) store<STREAM>(a.out + row + q + P * e, v[e].re);
+      if (hasB) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) store<STREAM>(a.out + row + N + q + P * e, v[e].im);
+      }
     } else {
       Cx<T>* out = reinterpret_cast<Cx<T>*>(a.out) + row;
-      store_line<E, P>(stream, out + q, [&](int e) { return v[e]; });
+      store_line<E, P>(S::streams(a.streamOut), out + q, [&](int e) { return v[e]; });
     }
   }
 }
@@ -1769,7 +1787,12 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
   for (int e = 0; e < E; ++e) uu[e] = a.xCol[q + P * e];
   for (int t = threadIdx.x; t < N; t += S::NT) twl[t] = a.twX[t];
   __syncthreads();
-  S::template fft<false, S::HALF_X>(v, region, wave, lane, twl);
+  Cx<T>* lr = S::xregion(region, wave, lane);
+  if constexpr (S::HALF_X) {
+    S::template fft<false, true>(v, region, wave, lane, twl);
+  } else {
+    wave_fft<T, N, false, 1, E>(v, lr, 1, q, twl);
+  }
   if (RC) {
     // Z = A + i B with A, B the spectra of the real rows a and b:
     // A[x] = (Z[x] + conj Z[N - x]) / 2, B[x] = -i (Z[x] - conj Z[N - x]) / 2.
@@ -1777,29 +1800,27 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
     // line's exchange region (wave-local; of a halved one, real and imaginary
     // parts in turn through registers).
     Cx<T> partner[S::HALF_X ? E : 1];
-    const Cx<T>* whole = S::xregion(region, wave, lane);
     wave_sync();
     if constexpr (S::HALF_X) {
-      T* lr = S::hregion(region, wave, lane);
+      T* half = S::hregion(region, wave, lane);
 #pragma unroll
-      for (int e = 0; e < E; ++e) lr[phys<float>(q + P * e)] = v[e].re;
+      for (int e = 0; e < E; ++e) half[phys<float>(q + P * e)] = v[e].re;
       wave_sync();
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int x = q + P * e;
-        partner[e].re = lr[phys<float>(x == 0 ? 0 : N - x)];
+        partner[e].re = half[phys<float>(x == 0 ? 0 : N - x)];
       }
       wave_sync();
 #pragma unroll
-      for (int e = 0; e < E; ++e) lr[phys<float>(q + P * e)] = v[e].im;
+      for (int e = 0; e < E; ++e) half[phys<float>(q + P * e)] = v[e].im;
       wave_sync();
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int x = q + P * e;
-        partner[e].im = lr[phys<float>(x == 0 ? 0 : N - x)];
+        partner[e].im = half[phys<float>(x == 0 ? 0 : N - x)];
       }
     } else {
-      Cx<T>* lr = S::xregion(region, wave, lane);
 #pragma unroll
       for (int e = 0; e < E; ++e) lr[phys<T>(q + P * e)] = v[e];
       wave_sync();
@@ -1810,12 +1831,7 @@ __device__ __forceinline__ void xsplit_forward_body(const FastArgs<T>& a, int bi
       for (int e = 0; e < E; ++e) {
         const int x = q + P * e;
         if (uu[e] < a.ncol) {
-          Cx<T> zp;
-          if constexpr (S::HALF_X) {
-            zp = partner[e];
-          } else {
-            zp = whole[phys<T>(x == 0 ? 0 : N - x)];
-          }
+          const Cx<T> zp = S::HALF_X ? partner[S::HALF_X ? e : 0] : lr[phys<T>(x == 0 ? 0 : N - x)];
           const T h = T(0.5);
           ya[uu[e]] = Cx<T>{h * (v[e].re + zp.re), h * (v[e].im - zp.im)};
           if (hasB) ya[a.pitchY + uu[e]] = Cx<T>{h * (v[e].im + zp.im), h * (zp.re - v[e].re)};
@@ -2041,9 +2057,9 @@ template <typename T, int N, bool RC>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_ysplit_backward(FastArgs<T> a) {
   ysplit_backward_body<T, N, RC>(a, blockIdx.x);
 }
-template <typename T, int N, bool RC>
+template <typename T, int N, bool RC, bool STREAM>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_xsplit_backward(FastArgs<T> a) {
-  xsplit_backward_body<T, N, RC>(a, blockIdx.x);
+  xsplit_backward_body<T, N, RC, STREAM>(a, blockIdx.x);
 }
 template <typename T, int N, bool RC, bool STREAM>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT)) k_xsplit_forward(FastArgs<T> a) {
@@ -2059,11 +2075,11 @@ __global__ void __launch_bounds__((SplitShape<T, N>::NT))
   const int t = blockIdx.x / perTransform;
   ysplit_backward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
-template <typename T, int N, bool RC, bool HALVES = true>
+template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_backward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_backward_body<T, N, RC, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_backward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
 }
 template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
@@ -2739,9 +2755,10 @@ void xsplit_n(bool forward, const FastArgs<T>& a, hipStream_t stream) {
                                        : k_xsplit_forward<T, NX, false, false>);
     split_launch<T, NX, false>(kernel, "k_xsplit_forward", blocks, stream, a);
   } else {
-    split_launch<T, NX, false>(
-        a.r2c ? k_xsplit_backward<T, NX, true> : k_xsplit_backward<T, NX, false>,
-        "k_xsplit_backward", blocks, stream, a);
+    auto kernel = !a.r2c ? k_xsplit_backward<T, NX, false, false>
+                  : S::streams(a.streamOut) ? k_xsplit_backward<T, NX, true, true>
+                                            : k_xsplit_backward<T, NX, true, false>;
+    split_launch<T, NX, false>(kernel, "k_xsplit_backward", blocks, stream, a);
   }
 }
 template <typename T, int NY, bool HALVES>
@@ -2764,14 +2781,14 @@ void ysplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans,
 }
 template <typename T, int NX, bool HALVES>
 void xsplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans, int ny, int nz,
-                    bool pastCache, hipStream_t stream) {
+                    size_t bytes, hipStream_t stream) {
   using S = SplitShape<T, NX, HALVES>;
   const int per = S::row_groups(ny, rc) * nz;
   if (forward) {
     auto kernel = rc ? k_xsplit_forward_batch<T, NX, true, true, HALVES>
                      : k_xsplit_forward_batch<T, NX, false, true, HALVES>;
     if constexpr (HALVES) {  // full regions: past the cache
-      if (!pastCache) {
+      if (bytes < kLastLevelCache) {
         kernel = rc ? k_xsplit_forward_batch<T, NX, true, false, HALVES>
                     : k_xsplit_forward_batch<T, NX, false, false, HALVES>;
       }
@@ -2780,11 +2797,14 @@ void xsplit_batch_n(bool forward, bool rc, const FastArgs<T>* batch, int ntrans,
         kernel, HALVES ? "k_xsplit_forward_batch" : "k_xsplit_forward_batch_full", per * ntrans,
         stream, batch, per);
   } else {
+    auto kernel = rc ? k_xsplit_backward_batch<T, NX, true, true, HALVES>
+                     : k_xsplit_backward_batch<T, NX, false, false, HALVES>;
+    if constexpr (HALVES) {
+      if (rc && bytes < kStreamBatch) kernel = k_xsplit_backward_batch<T, NX, true, false, HALVES>;
+    }
     split_launch<T, NX, false, HALVES>(
-        rc ? k_xsplit_backward_batch<T, NX, true, HALVES>
-           : k_xsplit_backward_batch<T, NX, false, HALVES>,
-        HALVES ? "k_xsplit_backward_batch" : "k_xsplit_backward_batch_full", per * ntrans, stream,
-        batch, per);
+        kernel, HALVES ? "k_xsplit_backward_batch" : "k_xsplit_backward_batch_full", per * ntrans,
+        stream, batch, per);
   }
 }
 template <typename T, int N, bool HALVES>
@@ -2792,7 +2812,7 @@ void split_batch_call(const SplitCall<T>& c) {
   if (c.y) {
     ysplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.nz, c.maxNcol, c.stream);
   } else {
-    xsplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.pastCache,
+    xsplit_batch_n<T, N, HALVES>(c.forward, c.rc, c.args, c.ntrans, c.ny, c.nz, c.bytes,
                                  c.stream);
   }
 }
@@ -2819,7 +2839,7 @@ void split_call(const SplitCall<T>& c) {
     }
   } else {
     if constexpr (SplitShape<T, N>::FULL_TOO) {
-      if (c.full) return split_batch_call<T, N, false>(c);
+      if (c.bytes >= kFullRegions) return split_batch_call<T, N, false>(c);
     }
     split_batch_call<T, N, true>(c);
   }
@@ -2861,8 +2881,7 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
     c.ny = ny;
     c.nz = nz;
     c.maxNcol = maxNcol;
-    c.full = bytes >= kFullRegions;
-    c.pastCache = bytes >= kLastLevelCache;
+    c.bytes = bytes;
     c.stream = stream;
     split_dispatch(c.y ? ny : nx, c);
   }
@@ -2921,7 +2940,8 @@ void launch_split_xy_batch(bool forward, bool r2c, int nx, int ny, const FastArg
 #define SPFFT_FAST_UNIT 0
 #endif
 #if SPFFT_FAST_UNIT == 0
-static_assert(kFullRegions >= kLastLevelCache, "full regions stream their loads");
+static_assert(kFullRegions >= kLastLevelCache && kFullRegions >= kStreamBatch,
+              "full regions stream");
 bool fixed_length(int n) { return square_length(n) || split_only_length(n); }
 SPFFT_INSTANTIATE_FAST_PLANE(double)
 #elif SPFFT_FAST_UNIT == 1
