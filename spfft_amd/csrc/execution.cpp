@@ -264,13 +264,20 @@ std::shared_ptr<TransformTables<T>> build_tables(const std::shared_ptr<IndexMap>
                   generic_candidate(map->dimX, map->dimY, map->dimZ);
   tb.generic = !useFast || tb.tryGeneric || (sizeof(T) == 4 && !r2c && !tb.fixedLengths);
   if (tb.generic) {
-    tb.entryValue = DeviceBuffer<int>::from_host(t.entryValue);
-    tb.entrySlot = DeviceBuffer<int>::from_host(t.entrySlot);
-    tb.stickY = DeviceBuffer<int>::from_host(t.stickY);
-    tb.stickCol = DeviceBuffer<int>::from_host(t.stickCol);
-    tb.colBegin = DeviceBuffer<int>::from_host(t.colBegin);
+    std::vector<int> all = t.entryValue;
+    auto append = [&](const std::vector<int>& v) {
+      const size_t at = all.size();
+      all.insert(all.end(), v.begin(), v.end());
+      return at;
+    };
+    tb.entrySlotAt = append(t.entrySlot);
+    tb.stickYAt = append(t.stickY);
+    tb.stickColAt = append(t.stickCol);
+    tb.colXAt = append(t.colX);
+    tb.colBeginAt = append(t.colBegin);
+    tb.stages = DeviceBuffer<int>::from_host(all);
   }
-  if (tb.generic || tb.split) tb.colX = DeviceBuffer<int>::from_host(t.colX);
+  if (tb.split) tb.colX = DeviceBuffer<int>::from_host(t.colX);
 
   if (useFast) {
     const int ny = map->dimY;
@@ -522,13 +529,14 @@ StageArgs<T> ExecutionGPU<T>::base_args() const {
   a.ncol = numCols_;
   a.r2c = map_->type == SPFFT_TRANS_R2C ? 1 : 0;
   a.zeroZeroStick = map_->zeroZeroStick;
-  a.entryValue = tab_->entryValue.data();
-  a.entrySlot = tab_->entrySlot.data();
+  const int* stages = tab_->stages.data();
+  a.entryValue = stages;
+  a.entrySlot = stages + tab_->entrySlotAt;
   a.stickBegin = tab_->stickBegin.data();
-  a.stickY = tab_->stickY.data();
-  a.stickCol = tab_->stickCol.data();
-  a.colX = tab_->colX.data();
-  a.colBegin = tab_->colBegin.data();
+  a.stickY = stages + tab_->stickYAt;
+  a.stickCol = stages + tab_->stickColAt;
+  a.colX = stages + tab_->colXAt;
+  a.colBegin = stages + tab_->colBeginAt;
   a.zbuf = reinterpret_cast<Cx<T>*>(grid_->sticks_gpu());
   a.ybuf = reinterpret_cast<Cx<T>*>(grid_->work_gpu());
   a.scale = scale_;

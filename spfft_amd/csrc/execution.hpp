@@ -46,7 +46,10 @@ struct TransformTables {
   int numCols = 0;
   int pitchT = 0;  // whole-plane batch kernels' tile pitch (0: not applicable)
   DeviceBuffer<Tw<T>> twX, twY, twZ;
-  DeviceBuffer<int> entryValue, entrySlot, stickBegin, stickY, stickCol, colX, colBegin;
+  DeviceBuffer<int> stickBegin, colX;
+  // tables of the generic kernels, one after the other in one allocation
+  DeviceBuffer<int> stages;
+  size_t entrySlotAt = 0, stickYAt = 0, stickColAt = 0, colXAt = 0, colBeginAt = 0;
   DeviceBuffer<int> stickAt;
   DeviceBuffer<int2> zEntries;
   DeviceBuffer<int4> zInfo;  // stick runs, when every stick is one run in user order
