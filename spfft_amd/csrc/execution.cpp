@@ -720,9 +720,9 @@ TuneChoice ExecutionGPU<T>::single_choice(bool forward, const FastArgs<T>& f, hi
   tune_record(key, c);
   if (tune_log_enabled()) {
     std::fprintf(stderr, "spfft_amd tune: %s N=%d Nz=%d %s %s, single transform, %d columns: z "
-                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f, matrix %.4f, generic (all "
-                 "stages) %.4f ms -> plane=%d zruns=%d\n", sizeof(T) == 8 ? "double" : "float", map_->dimX,
-                 map_->dimZ, map_->type == SPFFT_TRANS_R2C ? "R2C" : "C2C",
+                 "runs %.4f / entries %.4f ms; class-split %.4f, split stage %.4f, matrix %.4f, "
+                 "generic (all stages) %.4f ms -> plane=%d zruns=%d\n",
+                 sizeof(T) == 8 ? "double" : "float", map_->dimX, map_->dimZ, map_->type == SPFFT_TRANS_R2C ? "R2C" : "C2C",
                  forward ? "forward" : "backward", numCols_, zr, ze, fused, two, matrix, generic,
                  c.plane, c.zRuns);
   }

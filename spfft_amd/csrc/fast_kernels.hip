@@ -1541,7 +1541,8 @@ struct SplitShape {
       kLdsMax / (static_cast<size_t>(tw_offset<T>(FULL)) * sizeof(Cx<T>) + N * sizeof(Tw<T>) +
                  N * sizeof(Cx<T>)) * NW);
   static constexpr bool HALF_Y =
-      HALVES && sizeof(T) == 8 && N > 128 && dividing_schedule(N, L::E) && L::E % 2 == 0 && WAVES <= 12;
+      HALVES && sizeof(T) == 8 && N > 128 && dividing_schedule(N, L::E) && L::E % 2 == 0 &&
+      WAVES <= 12;
   static constexpr bool HALF_X = HALF_Y && N <= 256;
   // Lengths whose batches past kFullRegions take full regions in both kernels: those
   // without spare lanes, and with halved x kernels (192, 256; see kFullRegions).
@@ -2079,13 +2080,15 @@ template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_backward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_backward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_backward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch),
+                                                 blockIdx.x - t * perTransform);
 }
 template <typename T, int N, bool RC, bool STREAM, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
     k_xsplit_forward_batch(const FastArgs<T>* __restrict__ batch, int perTransform) {
   const int t = blockIdx.x / perTransform;
-  xsplit_forward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch), blockIdx.x - t * perTransform);
+  xsplit_forward_body<T, N, RC, STREAM, HALVES>(on_global(batch[t], batch),
+                                                blockIdx.x - t * perTransform);
 }
 template <typename T, int N, bool HALVES = true>
 __global__ void __launch_bounds__((SplitShape<T, N>::NT))
