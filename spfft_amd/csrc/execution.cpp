@@ -124,9 +124,10 @@ constexpr int kFromValues = 3000;
 //   250^3 FP64 634 / 381, 761 / 748, 1262 / 1305; FP32 447 / 249, 537 / 446, 858 / 734
 //   308^3 FP64 1068 / 1134, 1307 / 1294, 2152 / 2972; R2C FP64 782 / 676, 909 / 770,
 //     1331 / 1886
-// (the matrix kernels' work follows the square of the radius). Shorter lines all run
+// (the matrix kernels' work follows the square of the radius). Shorter free lines run
 // faster on the matrix kernels or even (radius 0.47 N: 143^3 FP64 199 / 184, FP32 174 /
-// 178; 143 x 160 x 160 257 / 228, 206 / 191), and so do sets with a prime factor above
+// 178; 143 x 160 x 160 257 / 228, 206 / 191), also beside fixed ones up to 256 (20 x 256
+// x 256 FP64 111 / 103, 65 x 192 x 192 180 / 149), and so do sets with a prime factor above
 // 13 (1.5 times at 17 x 320 x 320, radius 0.47 N; 2.6 to 47 at 221^3 to 319^3).
 bool generic_candidate(int nx, int ny, int nz) {
   auto smooth = [](int n) {
@@ -135,7 +136,8 @@ bool generic_candidate(int nx, int ny, int nz) {
     }
     return n == 1;
   };
-  return std::max({nx, ny, nz}) > 160 && smooth(nx) && smooth(ny) && smooth(nz);
+  auto is_long = [](int n) { return n > (fixed_length(n) ? 256 : 160); };
+  return (is_long(nx) || is_long(ny) || is_long(nz)) && smooth(nx) && smooth(ny) && smooth(nz);
 }
 
 // The plane family to run for `want` among those that serve the shape: the

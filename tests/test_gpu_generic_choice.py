@@ -1,7 +1,8 @@
-"""Sets with a long line that is not of a fixed length, all lengths without prime
-factors above 13: the first call times the generic kernels against the matrix kernels
-and keeps the faster (single transforms and batches), and either choice, once
-recorded, is the one that runs, also for one transform in a multi-transform call. Outputs are checked against the oracle each time.
+"""Sets with a long line, not all of fixed lengths and none with a prime factor above
+13: the first call times the generic kernels against the matrix kernels and keeps the
+faster (single transforms and batches), and either choice, once recorded, is the one
+that runs, also for one transform in a multi-transform call. Outputs are checked against
+the oracle each time.
 
 Each part runs in a fresh process, since the choices are per process. Tolerances: those
 of the generic kernels, 1e-12 (FP64) and 1e-5 (FP32)."""
@@ -32,7 +33,7 @@ from tests.workloads import complex_values
 for dims, r2c, precision, count, multi in (((245, 24, 18), False, "double", 1, False),
                                            ((20, 18, 250), True, "float", 1, False),
                                            ((16, 308, 24), True, "double", 3, True),
-                                           ((35, 176, 24), False, "float", 2, True),
+                                           ((35, 288, 24), False, "float", 2, True),
                                            ((245, 24, 18), False, "double", 1, True)):
     print("case", dims, count, flush=True)
     t = ellipsoid(dims, 0.4, r2c)
